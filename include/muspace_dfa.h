@@ -52,6 +52,7 @@
 #ifndef MUSPACE_DFA_H_
 #define MUSPACE_DFA_H_
 
+#include <stddef.h>
 #include <stdint.h>
 
 #include "muspace_msda.h"
@@ -78,6 +79,25 @@ MUSPACE_API int deformable_aggregation_backward_opt(
     float *grad_mc_ms_feat, float *grad_sampling_location, float *grad_weights, int64_t batch,
     int64_t num_cams, int64_t num_feat, int64_t num_embeds, int64_t num_scale,
     int64_t num_anchors, int64_t num_pts, int64_t num_groups, void *stream);
+
+/* The backward with grad_mc_ms_feat OVERWRITTEN (every element, zero where
+ * nothing samples it) instead of added to. Given a workspace of at least
+ * deformable_aggregation_backward_workspace_size bytes (0: the shape has no
+ * such path; NULL is then fine), each feature row's contributions are listed
+ * in it and summed once per row in float64, without atomics; else the
+ * gradient is zeroed and taken as by backward_opt. Nothing is kept in the
+ * workspace between calls. */
+MUSPACE_API size_t deformable_aggregation_backward_workspace_size(
+    int64_t batch, int64_t num_cams, int64_t num_feat, int64_t num_embeds, int64_t num_scale,
+    int64_t num_anchors, int64_t num_pts, int64_t num_groups);
+
+MUSPACE_API int deformable_aggregation_backward_ws(
+    const float *mc_ms_feat, const int32_t *spatial_shape, const int32_t *scale_start_index,
+    const float *sampling_location, const float *weights, const float *grad_output,
+    float *grad_mc_ms_feat, float *grad_sampling_location, float *grad_weights, int64_t batch,
+    int64_t num_cams, int64_t num_feat, int64_t num_embeds, int64_t num_scale,
+    int64_t num_anchors, int64_t num_pts, int64_t num_groups, void *workspace,
+    size_t workspace_bytes, void *stream);
 
 MUSPACE_API int deformable_aggregation_backward_base(
     const float *mc_ms_feat, const int32_t *spatial_shape, const int32_t *scale_start_index,

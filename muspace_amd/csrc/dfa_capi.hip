@@ -14,6 +14,7 @@
 
 #include <climits>
 #include <cstdint>
+#include <type_traits>
 
 #include "../../include/muspace_dfa.h"
 #include "capi_errors.hpp"
@@ -132,6 +133,14 @@ void launch_coarse(const int32_t *shape, const int32_t *start, const float *loc,
       shape, start, loc, weights, grad_out, grad_feat, d, budget, pair_log2, ns);
 }
 
+// Wavefronts per row of dfa_forward_rows: few rows give each of the 1024 SIMDs
+// few wavefronts with long serial pair walks, so a row's pairs are shared.
+// SparseDrive's 900 rows of one sample: 37.1, 31.2, 30.5 and 29.9 us at 2, 4, 8
+// and 16; its batch of 7,200 rows: 194.9, 185.8, 182.6 and 185.9 us.
+int forward_parts(int rows) {
+  return rows >= 8192 * 4 ? 1 : rows >= 8192 * 2 ? 2 : rows >= 2048 ? 8 : 16;
+}
+
 int forward_impl(const char *fn, bool optimized, const float *feat, const int32_t *shape,
                  const int32_t *start, const float *loc, const float *weights, float *out,
                  const DfaArgs &a, void *stream) {
@@ -145,29 +154,28 @@ int forward_impl(const char *fn, bool optimized, const float *feat, const int32_
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int nt = optimized ? row_slots(d) : 0;
   const int rows = d.batch * d.anchors;
-  // wavefronts per row of dfa_forward_rows (1, 2 or 4: one workgroup holds a
-  // row's parts): few rows give each SIMD few wavefronts with long serial
-  // pair walks, so a row's pairs are shared
-  const int parts = rows >= 8192 * 4 ? 1 : rows >= 8192 * 2 ? 2 : 4;
-  const int units = nt > 0 ? rows * parts : rows;
-  const int blocks = (units + dfa::kBlock / dfa::kWave - 1) / (dfa::kBlock / dfa::kWave);
+  const int parts = forward_parts(rows);
+  const int block = parts * dfa::kWave > dfa::kBlock ? parts * dfa::kWave : dfa::kBlock;
+  const int per_block = block / dfa::kWave;
+  const int blocks = (rows * parts + per_block - 1) / per_block;
+  const size_t lds = parts > 1 ? static_cast<size_t>(per_block) * d.embeds * sizeof(float) : 0;
   const uint32_t bytes = static_cast<uint32_t>(static_cast<uint64_t>(d.batch) * d.feat *
                                                d.embeds * 4u);
   switch (nt) {
     case 1:
-      dfa::dfa_forward_rows<1><<<blocks, dfa::kBlock, 0, st>>>(feat, bytes, shape, start, loc,
+      dfa::dfa_forward_rows<1><<<blocks, block, lds, st>>>(feat, bytes, shape, start, loc,
                                                                weights, out, d, parts);
       break;
     case 2:
-      dfa::dfa_forward_rows<2><<<blocks, dfa::kBlock, 0, st>>>(feat, bytes, shape, start, loc,
+      dfa::dfa_forward_rows<2><<<blocks, block, lds, st>>>(feat, bytes, shape, start, loc,
                                                                weights, out, d, parts);
       break;
     case 3:
-      dfa::dfa_forward_rows<3><<<blocks, dfa::kBlock, 0, st>>>(feat, bytes, shape, start, loc,
+      dfa::dfa_forward_rows<3><<<blocks, block, lds, st>>>(feat, bytes, shape, start, loc,
                                                                weights, out, d, parts);
       break;
     case 4:
-      dfa::dfa_forward_rows<4><<<blocks, dfa::kBlock, 0, st>>>(feat, bytes, shape, start, loc,
+      dfa::dfa_forward_rows<4><<<blocks, block, lds, st>>>(feat, bytes, shape, start, loc,
                                                                weights, out, d, parts);
       break;
     default:
@@ -178,6 +186,48 @@ int forward_impl(const char *fn, bool optimized, const float *feat, const int32_
   return check_launch(fn);
 }
 
+uint32_t feature_bytes(const dfa::Dims &d) {
+  return static_cast<uint32_t>(static_cast<uint64_t>(d.batch) * d.feat * d.embeds * 4u);
+}
+
+// Location and weight gradients by the row kernels; feature gradients with
+// device atomics too (kFeat), but for the maps that dfa_backward_coarse took
+// within `budget`.
+template <bool kFeat>
+void launch_backward_rows(int nt, const float *feat, const int32_t *shape, const int32_t *start,
+                          const float *loc, const float *weights, const float *grad_out,
+                          float *grad_feat, float *grad_loc, float *grad_weights,
+                          const dfa::Dims &d, int budget, hipStream_t st) {
+  const int rows = d.batch * d.anchors;
+  // wavefronts per row, as in the forward (SparseDrive's 7,200 rows: 205, 195,
+  // 205 and 236 us at 2, 4, 8 and 16; each part walks the row's locations)
+  const int parts = rows >= 8192 * 4 ? 1 : rows >= 8192 * 2 ? 2 : 4;
+  const int per_block = dfa::kBlock / dfa::kWave;
+  const int blocks = (rows * parts + per_block - 1) / per_block;
+  auto go = [&](auto slots) {
+    dfa::dfa_backward_rows<decltype(slots)::value, kFeat><<<blocks, dfa::kBlock, 0, st>>>(
+        feat, feature_bytes(d), shape, start, loc, weights, grad_out, grad_feat, grad_loc,
+        grad_weights, d, budget, parts);
+  };
+  switch (nt) {
+    case 1: go(std::integral_constant<int, 1>()); break;
+    case 2: go(std::integral_constant<int, 2>()); break;
+    case 3: go(std::integral_constant<int, 3>()); break;
+    default: go(std::integral_constant<int, 4>()); break;
+  }
+}
+
+void launch_backward_generic(const float *feat, const int32_t *shape, const int32_t *start,
+                             const float *loc, const float *weights, const float *grad_out,
+                             float *grad_feat, float *grad_loc, float *grad_weights,
+                             const dfa::Dims &d, hipStream_t st) {
+  const int64_t pairs = static_cast<int64_t>(d.batch) * d.anchors * d.pts * d.cams;
+  dfa::dfa_backward_generic<<<generic_blocks(pairs), dfa::kBlock, 0, st>>>(
+      feat, shape, start, loc, weights, grad_out, grad_feat, grad_loc, grad_weights, d);
+}
+
+// Feature gradients added to grad_feat without scratch: the small maps in LDS,
+// the others with the row kernels' atomics.
 int backward_impl(const char *fn, bool optimized, const float *feat, const int32_t *shape,
                   const int32_t *start, const float *loc, const float *weights,
                   const float *grad_out, float *grad_feat, float *grad_loc, float *grad_weights,
@@ -191,19 +241,14 @@ int backward_impl(const char *fn, bool optimized, const float *feat, const int32
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int nt = optimized ? row_slots(d) : 0;
-  const int rows = d.batch * d.anchors;
-  // wavefronts per row of dfa_backward_rows: few rows give each of the 1024
-  // SIMDs few wavefronts with long serial pair walks, so a row's pairs are
-  // shared (SparseDrive's 7,200 rows: backward call 929 -> 842 us at four)
-  const int parts = rows >= 8192 * 4 ? 1 : rows >= 8192 * 2 ? 2 : 4;
-  const int units = nt > 0 ? rows * parts : rows;
-  const int blocks = (units + dfa::kBlock / dfa::kWave - 1) / (dfa::kBlock / dfa::kWave);
-  const uint32_t bytes = static_cast<uint32_t>(static_cast<uint64_t>(d.batch) * d.feat *
-                                               d.embeds * 4u);
+  if (nt == 0) {
+    launch_backward_generic(feat, shape, start, loc, weights, grad_out, grad_feat, grad_loc,
+                            grad_weights, d, st);
+    return check_launch(fn);
+  }
   // the small maps' feature gradients summed in LDS first (they only add)
   int budget = 0, pair_log2 = 0;
-  const int cs = nt > 0 ? coarse_slice(d, loc, grad_out, budget, pair_log2) : 0;
-  switch (cs) {
+  switch (coarse_slice(d, loc, grad_out, budget, pair_log2)) {
     case 16:
       launch_coarse<16>(shape, start, loc, weights, grad_out, grad_feat, d, budget, pair_log2,
                         st);
@@ -218,37 +263,94 @@ int backward_impl(const char *fn, bool optimized, const float *feat, const int32
       budget = 0;
       break;
   }
+  launch_backward_rows<true>(nt, feat, shape, start, loc, weights, grad_out, grad_feat, grad_loc,
+                             grad_weights, d, budget, st);
+  return check_launch(fn);
+}
+
+// Scratch of the owner sums (deformable_aggregation_backward_ws).
+struct OwnerWorkspace {
+  size_t list, list_n, cursor, rows, contrib, bytes;
+};
+
+// False where the shape has no row kernel, or its contributions would pass
+// 32-bit offsets or 8 GiB: the gradients then come from the atomic kernels.
+bool plan_owner(const dfa::Dims &d, OwnerWorkspace &w) {
+  if (row_slots(d) == 0 || d.feat == 0) return false;
+  const uint64_t pairs = static_cast<uint64_t>(d.anchors) * d.pts;
+  const uint64_t cams = static_cast<uint64_t>(d.batch) * d.cams;
+  const uint64_t per_entry = pairs * d.cams * d.scales;  // Contribution::index
+  // dfa_sum_rows addresses an entry's weights and grad_out with 32-bit offsets
+  if (per_entry * d.groups * 4 > INT_MAX ||
+      static_cast<uint64_t>(d.anchors) * d.embeds * 4 > INT_MAX) {
+    return false;
+  }
+  const uint64_t most = 4u * per_entry * d.batch;
+  if (most > INT_MAX || cams * pairs > INT_MAX) return false;
+  size_t off = 0;
+  auto take = [&off](uint64_t bytes) {
+    const size_t at = off;
+    off += (bytes + 255) & ~uint64_t{255};
+    return at;
+  };
+  w.list = take(cams * pairs * sizeof(float4));
+  w.list_n = take(cams * sizeof(uint32_t));
+  w.cursor = take(sizeof(uint32_t));
+  w.rows = take(static_cast<uint64_t>(d.batch) * d.feat * sizeof(uint2));
+  w.contrib = take(most * sizeof(dfa::Contribution));
+  w.bytes = off;
+  return off <= (size_t{8} << 30);
+}
+
+// The backward with grad_feat overwritten: feature gradients by owner sums
+// when `workspace` holds them.
+int backward_ws_impl(const char *fn, const float *feat, const int32_t *shape,
+                     const int32_t *start, const float *loc, const float *weights,
+                     const float *grad_out, float *grad_feat, float *grad_loc,
+                     float *grad_weights, const DfaArgs &a, void *workspace,
+                     size_t workspace_bytes, void *stream) {
+  dfa::Dims d;
+  if (int rc = validate(fn, a, d)) return rc;
+  const int64_t n_feat = static_cast<int64_t>(d.batch) * d.feat * d.embeds;
+  const bool sampled = static_cast<int64_t>(d.batch) * d.anchors * d.pts * d.cams > 0;
+  if ((n_feat > 0 && !grad_feat) ||
+      (sampled && (!feat || !shape || !start || !loc || !grad_out || !grad_loc ||
+                   (!weights && d.scales > 0) || (!grad_weights && d.scales > 0)))) {
+    return fail(MUSPACE_EINVAL, "%s: null tensor pointer", fn);
+  }
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  OwnerWorkspace w;
+  if (!sampled || !plan_owner(d, w) || !workspace || workspace_bytes < w.bytes) {
+    if (n_feat > 0) {
+      dfa::dfa_zero<<<generic_blocks(n_feat), dfa::kBlock, 0, st>>>(grad_feat, n_feat);
+    }
+    if (!sampled) return check_launch(fn);
+    return backward_impl(fn, true, feat, shape, start, loc, weights, grad_out, grad_feat,
+                         grad_loc, grad_weights, a, stream);
+  }
+  unsigned char *ws = static_cast<unsigned char *>(workspace);
+  float4 *list = reinterpret_cast<float4 *>(ws + w.list);
+  uint32_t *list_n = reinterpret_cast<uint32_t *>(ws + w.list_n);
+  uint32_t *cursor = reinterpret_cast<uint32_t *>(ws + w.cursor);
+  uint2 *rows = reinterpret_cast<uint2 *>(ws + w.rows);
+  dfa::Contribution *contrib = reinterpret_cast<dfa::Contribution *>(ws + w.contrib);
+  const int nt = row_slots(d);
+  dfa::dfa_list_active<<<d.batch * d.cams, dfa::kListBlock, 0, st>>>(loc, list, list_n, cursor, d);
+  const int ranges = (d.feat + dfa::kRangeRows - 1) / dfa::kRangeRows;
+  dfa::dfa_list_rows<<<d.batch * ranges, dfa::kRangeBlock, 0, st>>>(
+      shape, start, list, list_n, cursor, rows, contrib, d, ranges);
+  launch_backward_rows<false>(nt, feat, shape, start, loc, weights, grad_out, nullptr, grad_loc,
+                              grad_weights, d, 0, st);
+  const int per_entry = (d.feat + dfa::kSumRows - 1) / dfa::kSumRows;
+  auto sum = [&](auto slots) {
+    dfa::dfa_sum_rows<decltype(slots)::value><<<d.batch * per_entry, dfa::kBlock, 0, st>>>(
+        weights, grad_out, rows, contrib, grad_feat, d, per_entry);
+  };
   switch (nt) {
-    case 1:
-      dfa::dfa_backward_rows<1><<<blocks, dfa::kBlock, 0, st>>>(feat, bytes, shape, start, loc,
-                                                                weights, grad_out, grad_feat,
-                                                                grad_loc, grad_weights, d, budget,
-                                                                parts);
-      break;
-    case 2:
-      dfa::dfa_backward_rows<2><<<blocks, dfa::kBlock, 0, st>>>(feat, bytes, shape, start, loc,
-                                                                weights, grad_out, grad_feat,
-                                                                grad_loc, grad_weights, d, budget,
-                                                                parts);
-      break;
-    case 3:
-      dfa::dfa_backward_rows<3><<<blocks, dfa::kBlock, 0, st>>>(feat, bytes, shape, start, loc,
-                                                                weights, grad_out, grad_feat,
-                                                                grad_loc, grad_weights, d, budget,
-                                                                parts);
-      break;
-    case 4:
-      dfa::dfa_backward_rows<4><<<blocks, dfa::kBlock, 0, st>>>(feat, bytes, shape, start, loc,
-                                                                weights, grad_out, grad_feat,
-                                                                grad_loc, grad_weights, d, budget,
-                                                                parts);
-      break;
-    default:
-      dfa::dfa_backward_generic<<<generic_blocks(static_cast<int64_t>(rows) * d.pts * d.cams),
-                                  dfa::kBlock, 0, st>>>(feat, shape, start, loc, weights,
-                                                        grad_out, grad_feat, grad_loc,
-                                                        grad_weights, d);
-      break;
+    case 1: sum(std::integral_constant<int, 1>()); break;
+    case 2: sum(std::integral_constant<int, 2>()); break;
+    case 3: sum(std::integral_constant<int, 3>()); break;
+    default: sum(std::integral_constant<int, 4>()); break;
   }
   return check_launch(fn);
 }
@@ -294,6 +396,34 @@ int deformable_aggregation_backward_opt(
   return backward_impl("deformable_aggregation_backward_opt", true, mc_ms_feat, spatial_shape,
                        scale_start_index, sampling_location, weights, grad_output,
                        grad_mc_ms_feat, grad_sampling_location, grad_weights, a, stream);
+}
+
+size_t deformable_aggregation_backward_workspace_size(int64_t batch, int64_t num_cams,
+                                                      int64_t num_feat, int64_t num_embeds,
+                                                      int64_t num_scale, int64_t num_anchors,
+                                                      int64_t num_pts, int64_t num_groups) {
+  const DfaArgs a{batch, num_cams, num_feat, num_embeds, num_scale, num_anchors, num_pts,
+                  num_groups};
+  dfa::Dims d;
+  OwnerWorkspace w;
+  if (validate("deformable_aggregation_backward_workspace_size", a, d) != 0) return 0;
+  if (static_cast<int64_t>(d.batch) * d.anchors * d.pts * d.cams == 0) return 0;
+  return plan_owner(d, w) ? w.bytes : 0;
+}
+
+int deformable_aggregation_backward_ws(
+    const float *mc_ms_feat, const int32_t *spatial_shape, const int32_t *scale_start_index,
+    const float *sampling_location, const float *weights, const float *grad_output,
+    float *grad_mc_ms_feat, float *grad_sampling_location, float *grad_weights, int64_t batch,
+    int64_t num_cams, int64_t num_feat, int64_t num_embeds, int64_t num_scale,
+    int64_t num_anchors, int64_t num_pts, int64_t num_groups, void *workspace,
+    size_t workspace_bytes, void *stream) {
+  const DfaArgs a{batch, num_cams, num_feat, num_embeds, num_scale, num_anchors, num_pts,
+                  num_groups};
+  return backward_ws_impl("deformable_aggregation_backward_ws", mc_ms_feat, spatial_shape,
+                          scale_start_index, sampling_location, weights, grad_output,
+                          grad_mc_ms_feat, grad_sampling_location, grad_weights, a, workspace,
+                          workspace_bytes, stream);
 }
 
 int deformable_aggregation_backward_base(

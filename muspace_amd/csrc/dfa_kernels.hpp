@@ -17,13 +17,14 @@
 // (/root/reference/csrc/deformable_aggregation/deformable_aggregation_musa.mu:39-160,304-430)
 // and the PyTorch reference (/root/reference/mu_space/ops/deformable_aggregation.py:88-158).
 //
-// Row kernels (C = 64*NT channels, NT <= 4): one to four wavefronts per
-// (batch, anchor) row; lane i owns channels i, i+64, ... so every gather,
-// atomic and store of a corner row is a contiguous 256-byte access. The lanes
+// Row kernels (C = 64*NT channels, NT <= 4): one to sixteen wavefronts per
+// (batch, anchor) row; a lane owns NT channels (Lanes), so a corner row of C
+// channels is one contiguous load instruction of 4*NT bytes a lane. The lanes
 // load the locations of 64 (pt, cam) pairs at once and ballot the active ones;
 // each wavefront then walks only its share of the active pairs, whose geometry
-// is uniform (read from the owning lane). Corner loads are unconditional raw buffer loads: a corner outside its
-// map gets an out-of-range offset, which reads zero.
+// is uniform (read from the owning lane). Corner loads are unconditional raw
+// buffer loads: a corner outside its map gets an out-of-range offset, which
+// reads zero.
 //
 // Generic kernels (any C and groups) exist for shape coverage, not speed.
 #pragma once
@@ -132,8 +133,9 @@ __device__ __forceinline__ bool active(float x, float y) {
   return x > 0.0f && x < 1.0f && y > 0.0f && y < 1.0f;  // NaN is inactive
 }
 
-__device__ __forceinline__ float buffer_load4(__amdgpu_buffer_rsrc_t r, uint32_t offset) {
-  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, offset, 0, 0));
+__device__ __forceinline__ float buffer_load4(__amdgpu_buffer_rsrc_t r, uint32_t offset,
+                                              uint32_t uniform = 0u) {
+  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, offset, uniform, 0));
 }
 
 // Sum over the wavefront, every lane receiving it (DPP inside the 16-lane
@@ -146,38 +148,147 @@ __device__ __forceinline__ float segment_sum(float v, int width) {
   return msda::group_sum_sel(v, width);
 }
 
-// Forward, one (batch, anchor) row over `parts` (1, 2 or 4) wavefronts of one
-// workgroup: the row's active pairs are dealt round-robin by their rank among
-// the active pairs, and the parts' partial rows are summed through LDS by
-// part 0, which adds the row to `out`.
+// A lane's NT channels of a row (C = 64 * NT). Packed (NT = 1, 2 and 4): the
+// consecutive channels NT * lane .., all in one weight group (a group is a power
+// of two of at least 8 channels there), so a corner row is one 4*NT-byte load a
+// lane and a group's sum starts with the lane's own channels. Else channels
+// lane, lane + 64, ...: NT = 3 (C = 192, groups of 64 or 192 channels), and
+// where a row takes device atomics, which want whole lines per instruction.
+typedef float f32x2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int NT, bool kPacked_ = NT != 3>
+struct Lanes {
+  static constexpr bool kPacked = kPacked_;
+  static_assert(!kPacked || NT != 3, "a lane's packed channels are in one group");
+  static constexpr int kGroups = kPacked ? 1 : NT;  // weights a lane needs per scale
+  static __device__ __forceinline__ int channel(int lane, int t) {
+    return kPacked ? lane * NT + t : t * kWave + lane;
+  }
+  // the lane's channels of the row at byte offset `row` (+ `uniform`, a scalar)
+  static __device__ __forceinline__ void gather(__amdgpu_buffer_rsrc_t r, uint32_t row, int lane,
+                                                float (&v)[NT], uint32_t uniform = 0u) {
+    if constexpr (kPacked && NT == 4) {
+      const msda::u32x4 w =
+          __builtin_amdgcn_raw_buffer_load_b128(r, row + lane * 16u, uniform, 0);
+      v[0] = __uint_as_float(w.x);
+      v[1] = __uint_as_float(w.y);
+      v[2] = __uint_as_float(w.z);
+      v[3] = __uint_as_float(w.w);
+    } else if constexpr (kPacked && NT == 2) {
+      const auto w = __builtin_amdgcn_raw_buffer_load_b64(r, row + lane * 8u, uniform, 0);
+      v[0] = __uint_as_float(w[0]);
+      v[1] = __uint_as_float(w[1]);
+    } else {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) v[t] = buffer_load4(r, row + (t * kWave + lane) * 4u, uniform);
+    }
+  }
+  // ... of a dense row (4-byte alignment suffices)
+  static __device__ __forceinline__ void load(const float *row, int lane, float (&v)[NT]) {
+    if constexpr (kPacked && NT == 4) {
+      const f32x4 w = *reinterpret_cast<const f32x4 *>(row + lane * 4);
+      v[0] = w.x;
+      v[1] = w.y;
+      v[2] = w.z;
+      v[3] = w.w;
+    } else if constexpr (kPacked && NT == 2) {
+      const f32x2 w = *reinterpret_cast<const f32x2 *>(row + lane * 2);
+      v[0] = w.x;
+      v[1] = w.y;
+    } else {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) v[t] = row[t * kWave + lane];
+    }
+  }
+  static __device__ __forceinline__ void store_nt(float *row, int lane, const float (&v)[NT]) {
+    if constexpr (kPacked && NT == 4) {
+      __builtin_nontemporal_store(f32x4{v[0], v[1], v[2], v[3]},
+                                  reinterpret_cast<f32x4 *>(row + lane * 4));
+    } else if constexpr (kPacked && NT == 2) {
+      __builtin_nontemporal_store(f32x2{v[0], v[1]}, reinterpret_cast<f32x2 *>(row + lane * 2));
+    } else {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) __builtin_nontemporal_store(v[t], row + t * kWave + lane);
+    }
+  }
+  static __device__ __forceinline__ void store(float *row, int lane, const float (&v)[NT]) {
+    if constexpr (kPacked && NT == 4) {
+      *reinterpret_cast<f32x4 *>(row + lane * 4) = f32x4{v[0], v[1], v[2], v[3]};
+    } else if constexpr (kPacked && NT == 2) {
+      *reinterpret_cast<f32x2 *>(row + lane * 2) = f32x2{v[0], v[1]};
+    } else {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) row[t * kWave + lane] = v[t];
+    }
+  }
+};
+
+// A pair's corner rows and weights are loaded kScaleRun scales at a time before
+// either is used, so one memory latency covers them.
+constexpr int kScaleRun = 2;
+constexpr int kMaxParts = 16;  // wavefronts per (batch, anchor) row
+
+// The loads of one run of scales of one pair at (x, y): corner rows (zeros
+// outside the map and for scales past the last) and the lane's weights.
+template <int NT, typename L>
+__device__ __forceinline__ void load_run(__amdgpu_buffer_rsrc_t rf, uint32_t batch_row,
+                                         const View *cv, const float *wp, const int (&grp)[NT],
+                                         float x, float y, int s0, int lane, const Dims &d,
+                                         float (&val)[kScaleRun][4][NT],
+                                         float (&wv)[kScaleRun][L::kGroups]) {
+  constexpr int C = NT * kWave;
+#pragma unroll
+  for (int j = 0; j < kScaleRun; ++j) {
+    const int s = min(s0 + j, d.scales - 1);
+    const View v = cv[s];
+    const Tap tp = make_tap(x, y, v);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const bool ok = s0 + j < d.scales && v.h > 0 && tp.cell[k] >= 0;
+      L::gather(
+          rf, ok ? (batch_row + static_cast<uint32_t>(v.start + tp.cell[k])) * (C * 4u) : kOobOffset,
+          lane, val[j][k]);
+    }
+#pragma unroll
+    for (int t = 0; t < L::kGroups; ++t) wv[j][t] = wp[s * d.groups + grp[t]];
+  }
+}
+
+// Forward, one (batch, anchor) row over `parts` (a power of two up to 16)
+// wavefronts of one workgroup: the row's active pairs are dealt round-robin by
+// their rank among the active pairs, and the parts' partial rows are summed
+// through LDS by part 0, which adds the row to `out`.
 template <int NT>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kMaxParts * kWave)
     dfa_forward_rows(const float *__restrict__ feat, uint32_t feat_bytes,
                      const int32_t *__restrict__ shape, const int32_t *__restrict__ start,
                      const float *__restrict__ loc, const float *__restrict__ weights,
                      float *__restrict__ out, Dims d, int parts) {
+  using L = Lanes<NT>;
   constexpr int C = NT * kWave;
   __shared__ View views[kMaxViews];
-  __shared__ float partial[kBlock / kWave][C];
+  extern __shared__ float partial[];  // [wavefronts][C] when parts > 1
   stage_views(views, shape, start, d);
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const int unit = msda::xcd_logical_block(blockIdx.x, gridDim.x) * (kBlock / kWave) + wave;
-  const int row = unit / parts, part = unit & (parts - 1);  // parts: 1, 2 or 4
+  const int unit = msda::xcd_logical_block(blockIdx.x, gridDim.x) * (blockDim.x / kWave) + wave;
+  const int row = unit / parts, part = unit & (parts - 1);
   const bool live = row < d.batch * d.anchors;  // every wavefront reaches the barrier below
   const int b = live ? row / d.anchors : 0;
   const int cpg = C / d.groups;
   const __amdgpu_buffer_rsrc_t rf = msda::make_rsrc(feat, feat_bytes);
   int grp[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) grp[t] = (t * kWave + lane) / cpg;
   float acc[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = 0.0f;
+  for (int t = 0; t < NT; ++t) {
+    grp[t] = L::channel(lane, t) / cpg;
+    acc[t] = 0.0f;
+  }
 
   const int pairs = d.pts * d.cams, sg = d.scales * d.groups;
   const float *loc_row = loc + static_cast<size_t>(row) * pairs * 2;
   const float *w_row = weights + static_cast<size_t>(row) * pairs * sg;
-  const uint32_t batch_base = static_cast<uint32_t>(b) * static_cast<uint32_t>(d.feat);
+  const uint32_t batch_row = static_cast<uint32_t>(b) * static_cast<uint32_t>(d.feat);
   const uint64_t below = (uint64_t{1} << lane) - 1;
   int seen = 0;  // active pairs of the row before this run of 64
   for (int base = 0; live && base < pairs; base += kWave) {
@@ -195,58 +306,54 @@ __global__ void __launch_bounds__(kBlock)
       const float y = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ly), l));
       const int pair = base + l, cam = pair % d.cams;
       const float *wp = w_row + static_cast<size_t>(pair) * sg;
-#pragma unroll 2
-      for (int s = 0; s < d.scales; ++s) {
-        const View v = views[cam * d.scales + s];
-        const Tap tp = make_tap(x, y, v);
-        float val[4][NT];
+      const View *cv = views + cam * d.scales;
+      for (int s0 = 0; s0 < d.scales; s0 += kScaleRun) {
+        float val[kScaleRun][4][NT], wv[kScaleRun][L::kGroups];
+        load_run<NT, L>(rf, batch_row, cv, wp, grp, x, y, s0, lane, d, val, wv);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const bool ok = v.h > 0 && tp.cell[k] >= 0;
-          const uint32_t row_off =
-              ok ? (batch_base + static_cast<uint32_t>(v.start + tp.cell[k])) * (C * 4u)
-                 : kOobOffset;
+        for (int j = 0; j < kScaleRun; ++j) {
+          if (s0 + j >= d.scales) break;  // uniform
+          const Tap tp = make_tap(x, y, cv[s0 + j]);
 #pragma unroll
-          for (int t = 0; t < NT; ++t) val[k][t] = buffer_load4(rf, row_off + (t * kWave + lane) * 4u);
-        }
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          const float wg = wp[s * d.groups + grp[t]];
-          acc[t] += (tp.w[0] * val[0][t] + tp.w[1] * val[1][t] + tp.w[2] * val[2][t] +
-                     tp.w[3] * val[3][t]) * wg;
+          for (int t = 0; t < NT; ++t) {
+            acc[t] += (tp.w[0] * val[j][0][t] + tp.w[1] * val[j][1][t] + tp.w[2] * val[j][2][t] +
+                       tp.w[3] * val[j][3][t]) * wv[j][L::kPacked ? 0 : t];
+          }
         }
       }
     }
   }
   if (parts > 1) {  // uniform over the workgroup
-    if (part > 0) {
-#pragma unroll
-      for (int t = 0; t < NT; ++t) partial[wave][t * kWave + lane] = acc[t];
-    }
+    if (part > 0) L::store(partial + wave * C, lane, acc);
     __syncthreads();
     if (part > 0) return;
     for (int w = wave + 1; w < wave + parts; ++w) {
+      float p[NT];
+      L::load(partial + w * C, lane, p);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t] += partial[w][t * kWave + lane];
+      for (int t = 0; t < NT; ++t) acc[t] += p[t];
     }
   }
   if (!live) return;
-  float *o = out + static_cast<size_t>(row) * C + lane;
+  float *o = out + static_cast<size_t>(row) * C;
+  float old[NT];
+  L::load(o, lane, old);
 #pragma unroll
-  for (int t = 0; t < NT; ++t) o[t * kWave] += acc[t];
+  for (int t = 0; t < NT; ++t) old[t] += acc[t];
+  L::store(o, lane, old);
 }
 
 // Backward, one (batch, anchor) row split over `parts` wavefronts: the row's
 // active pairs are dealt round-robin (by their rank among the active pairs)
 // so that every wavefront of the row gets a near-equal share; a skipped
 // pair's zero gradients go to the wavefront `pair % parts`. Location and
-// weight gradients are per pair and feature gradients are atomics, so the
-// parts need no reduction. A pair's corner rows and weights are loaded two
-// scales at a time before either is used, so one memory latency covers two
-// scales (four scales at once cost registers and occupancy: slower).
-constexpr int kScaleRun = 2;
-
-template <int NT>
+// weight gradients are per pair and feature gradients are atomics (kFeat) or
+// left to dfa_sum_rows, so the parts need no reduction.
+//
+// A lane sums g times the sample and g times its slopes over its channels
+// first; the weight gradient of a group is then one sum over the group's lanes
+// per scale, and the location gradient one wavefront sum per pair.
+template <int NT, bool kFeat>
 __global__ void __launch_bounds__(kBlock)
     dfa_backward_rows(const float *__restrict__ feat, uint32_t feat_bytes,
                       const int32_t *__restrict__ shape, const int32_t *__restrict__ start,
@@ -254,27 +361,27 @@ __global__ void __launch_bounds__(kBlock)
                       const float *__restrict__ grad_out, float *__restrict__ grad_feat,
                       float *__restrict__ grad_loc, float *__restrict__ grad_weights, Dims d,
                       int coarse_budget, int parts) {
+  using L = Lanes<NT, NT != 3 && !kFeat>;
   constexpr int C = NT * kWave;
   __shared__ View views[kMaxViews];
   stage_views(views, shape, start, d);
-  mark_coarse(views, d, coarse_budget);  // maps whose feature gradients another kernel sums
+  if constexpr (kFeat) mark_coarse(views, d, coarse_budget);  // maps whose feature gradients another kernel sums
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int unit = msda::xcd_logical_block(blockIdx.x, gridDim.x) * (kBlock / kWave) + wave;
-  const int row = unit / parts, part = unit & (parts - 1);  // parts: 1, 2 or 4
+  const int row = unit / parts, part = unit & (parts - 1);  // parts: a power of two up to 16
   if (row >= d.batch * d.anchors) return;  // no barrier follows
   const int b = row / d.anchors;
   const int cpg = C / d.groups;
-  const int seg = cpg < kWave ? cpg : kWave;  // lanes summed for one group's weight gradient
-  const int tpg = cpg / seg;                  // channel slots per group (cpg > 64)
+  // lanes summed for one group's weight gradient; NT = 3 has one sum per
+  // channel slot, tpg of them a group
+  const int seg = L::kPacked ? cpg / NT : min(cpg, kWave);
+  const int tpg = L::kPacked ? 1 : cpg / seg;
   const __amdgpu_buffer_rsrc_t rf = msda::make_rsrc(feat, feat_bytes);
   int grp[NT];
   float g[NT];
-  const float *go = grad_out + static_cast<size_t>(row) * C + lane;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    grp[t] = (t * kWave + lane) / cpg;
-    g[t] = go[t * kWave];
-  }
+  for (int t = 0; t < NT; ++t) grp[t] = L::channel(lane, t) / cpg;
+  L::load(grad_out + static_cast<size_t>(row) * C, lane, g);
 
   const int pairs = d.pts * d.cams, sg = d.scales * d.groups;
   const float *loc_row = loc + static_cast<size_t>(row) * pairs * 2;
@@ -285,8 +392,9 @@ __global__ void __launch_bounds__(kBlock)
   const uint32_t batch_row = static_cast<uint32_t>(b) * static_cast<uint32_t>(d.feat);
   const uint64_t below = (uint64_t{1} << lane) - 1;
   const int sgd = sg > 0 ? sg : 1;  // no scales: nothing is zeroed
-  const int lane_p = lane / sgd, lane_j = lane - lane_p * sgd;  // element `lane` of a run
-  const int step_p = kWave / sgd, step_j = kWave - step_p * sgd;
+  const int own_n = sg > 0 ? kWave / parts : 0;  // pairs of a run this part zeroes if skipped
+  const int lane_i = lane / sgd, lane_j = lane - lane_i * sgd;
+  const int step_i = kWave / sgd, step_j = kWave - step_i * sgd;
   int seen = 0;  // active pairs of the row before this run of 64
   for (int base = 0; base < pairs; base += kWave) {
     const int n = min(kWave, pairs - base);
@@ -297,17 +405,17 @@ __global__ void __launch_bounds__(kBlock)
     const int owner = (on ? seen + __builtin_popcountll(act & below) : pi) & (parts - 1);
     const uint64_t own = __ballot(lane < n && owner == part);
     seen += __builtin_popcountll(act);
-    // weight gradients of skipped pairs are zero: element e = p * sg + j of
-    // the run, (p, j) stepped by kWave elements per pass (no division inside)
-    for (int e = lane, p = lane_p, j = lane_j; e < n * sg; e += kWave) {
-      if (!((act >> p) & 1) && ((base + p) & (parts - 1)) == part) {
-        gw_row[static_cast<size_t>(base) * sg + e] = 0.0f;
-      }
-      p += step_p;
+    // weight gradients of skipped pairs are zero: element j of this part's
+    // i-th pair p = part + i * parts of the run (base is a multiple of parts),
+    // (i, j) stepped by kWave elements per pass (no division inside)
+    for (int i = lane_i, j = lane_j; i < own_n;) {
+      const int p = part + i * parts;
+      if (p < n && !((act >> p) & 1)) gw_row[static_cast<size_t>(base + p) * sg + j] = 0.0f;
+      i += step_i;
       j += step_j;
       if (j >= sg) {
         j -= sg;
-        ++p;
+        ++i;
       }
     }
     float my_gx = 0.0f, my_gy = 0.0f;  // location gradient of this lane's pair
@@ -323,75 +431,62 @@ __global__ void __launch_bounds__(kBlock)
       const View *cv = views + cam * d.scales;
       float gx = 0.0f, gy = 0.0f;
       for (int s0 = 0; s0 < d.scales; s0 += kScaleRun) {
-        // every load of the run first (scales past the last read nothing)
-        float val[kScaleRun][4][NT];
-        float wv[kScaleRun][NT];
-#pragma unroll
-        for (int j = 0; j < kScaleRun; ++j) {
-          const int s = min(s0 + j, d.scales - 1);
-          const View v = cv[s];
-          const Tap tp = make_tap(x, y, v);
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const bool ok = s0 + j < d.scales && v.h > 0 && tp.cell[k] >= 0;
-            const uint32_t row_off =
-                ok ? (batch_row + static_cast<uint32_t>(v.start + tp.cell[k])) * (C * 4u)
-                   : kOobOffset;
-#pragma unroll
-            for (int t = 0; t < NT; ++t) {
-              val[j][k][t] = buffer_load4(rf, row_off + (t * kWave + lane) * 4u);
-            }
-          }
-#pragma unroll
-          for (int t = 0; t < NT; ++t) wv[j][t] = wp[s * d.groups + grp[t]];
-        }
+        float val[kScaleRun][4][NT], wv[kScaleRun][L::kGroups];
+        load_run<NT, L>(rf, batch_row, cv, wp, grp, x, y, s0, lane, d, val, wv);
 #pragma unroll
         for (int j = 0; j < kScaleRun; ++j) {
           const int s = s0 + j;
           if (s >= d.scales) break;  // uniform
           const View v = cv[s];
           const Tap tp = make_tap(x, y, v);
-          float gwt[NT];
-          float top[NT];
+          float gwt[L::kGroups];
+          // per weight the lane holds, g times the sample and its slopes, summed
+          // over the channels under that weight (all the lane's, or one)
 #pragma unroll
-          for (int t = 0; t < NT; ++t) {
-            top[t] = g[t] * wv[j][t];
-            const float q0 = val[j][0][t], q1 = val[j][1][t], q2 = val[j][2][t],
-                        q3 = val[j][3][t];
-            gwt[t] = g[t] * (tp.w[0] * q0 + tp.w[1] * q1 + tp.w[2] * q2 + tp.w[3] * q3);
-            const float dh = -tp.hw * q0 - tp.lw * q1 + tp.hw * q2 + tp.lw * q3;
-            const float dw = -tp.hh * q0 + tp.hh * q1 - tp.lh * q2 + tp.lh * q3;
-            gx += static_cast<float>(v.w) * dw * top[t];
-            gy += static_cast<float>(v.h) * dh * top[t];
+          for (int u = 0; u < L::kGroups; ++u) {
+            gwt[u] = 0.0f;
+            float sw = 0.0f, sh = 0.0f;
+#pragma unroll
+            for (int t = L::kPacked ? 0 : u; t <= (L::kPacked ? NT - 1 : u); ++t) {
+              const float q0 = val[j][0][t], q1 = val[j][1][t], q2 = val[j][2][t],
+                          q3 = val[j][3][t];
+              gwt[u] += g[t] * (tp.w[0] * q0 + tp.w[1] * q1 + tp.w[2] * q2 + tp.w[3] * q3);
+              sw += g[t] * (-tp.hh * q0 + tp.hh * q1 - tp.lh * q2 + tp.lh * q3);
+              sh += g[t] * (-tp.hw * q0 - tp.lw * q1 + tp.hw * q2 + tp.lw * q3);
+            }
+            gx += static_cast<float>(v.w) * sw * wv[j][u];
+            gy += static_cast<float>(v.h) * sh * wv[j][u];
           }
-          // feature gradient: one contiguous 256-byte atomic per corner and slot
+          // feature gradient: one contiguous atomic per corner and slot
           // (maps summed by dfa_backward_coarse are left to it)
-          if (v.lds < 0 && v.h > 0) {  // uniform across the wavefront
+          if (kFeat && v.lds < 0 && v.h > 0) {  // uniform across the wavefront
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
               if (tp.cell[k] >= 0) {
-                float *dst =
-                    grad_feat + batch_elem + static_cast<size_t>(v.start + tp.cell[k]) * C + lane;
+                float *dst = grad_feat + batch_elem + static_cast<size_t>(v.start + tp.cell[k]) * C;
 #pragma unroll
-                for (int t = 0; t < NT; ++t) unsafeAtomicAdd(dst + t * kWave, tp.w[k] * top[t]);
+                for (int t = 0; t < NT; ++t) {
+                  unsafeAtomicAdd(dst + L::channel(lane, t),
+                                  tp.w[k] * (g[t] * wv[j][L::kPacked ? 0 : t]));
+                }
               }
             }
           }
           // weight gradient of each group: sum over its channels
           if (tpg == 1) {
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-              const float sum = segment_sum(gwt[t], seg);
-              if ((lane & (seg - 1)) == 0) gwp[s * d.groups + grp[t]] = sum;
+            for (int u = 0; u < L::kGroups; ++u) {
+              const float sum = segment_sum(gwt[u], seg);
+              if ((lane & (seg - 1)) == 0) gwp[s * d.groups + grp[u]] = sum;
             }
           } else {
 #pragma unroll
-            for (int t = 0; t < NT; ++t) gwt[t] = wave_sum(gwt[t]);
+            for (int u = 0; u < L::kGroups; ++u) gwt[u] = wave_sum(gwt[u]);
             if (lane == 0) {
               for (int gi = 0; gi < d.groups; ++gi) {
                 float sum = 0.0f;
 #pragma unroll
-                for (int t = 0; t < NT; ++t) sum += t / tpg == gi ? gwt[t] : 0.0f;
+                for (int u = 0; u < L::kGroups; ++u) sum += u / tpg == gi ? gwt[u] : 0.0f;
                 gwp[s * d.groups + gi] = sum;
               }
             }
@@ -409,6 +504,293 @@ __global__ void __launch_bounds__(kBlock)
       gl_row[2 * (base + lane)] = my_gx;
       gl_row[2 * (base + lane) + 1] = my_gy;
     }
+  }
+}
+
+// ------------------------------------------------- feature gradients ---
+//
+// Sums by owner: every feature row's contributions are listed (a counting sort
+// by row) and one wavefront run sums them in registers and writes the row once,
+// so the gradient takes no atomics and no zero fill: dfa_list_active ->
+// dfa_list_rows -> dfa_sum_rows. SparseDrive's training batch (8 x 900
+// anchors, 718 k feature rows of 1 KB, 1.67 M contributions): 13 + 37 + 261 us
+// and 195 us for the row kernel without atomics, against a zero fill of 735 MB,
+// 433 us for LDS sums of the small maps and 416 us for the row kernel with
+// atomics on the largest: training call 1120 -> 675 us. dfa_sum_rows writes
+// 735 MB (110 us of it: 150 us without its stores) and gathers each
+// contribution's 1 KB grad_out row from L2; its wavefronts wait on that chain
+// (row table, contributions, rows). Persistent workgroups with the tables
+// loaded blocks ahead were slower (281-301 us: a wavefront's loads then wait for
+// its earlier stores, which complete in order), and so were 32 rows a
+// workgroup (280 us) and eight rows requested at a time (273 us).
+//
+// Sums are float64 over the exact products w_corner * (grad_out * weight), the
+// operands float32, and are rounded once, so their order (which the counting
+// sort leaves open) does not show.
+
+constexpr int kListBlock = 1024;
+constexpr int kRangeRows = 2048;  // feature rows counted by one workgroup of dfa_list_rows
+constexpr int kRangeBlock = 512;
+constexpr int kSumRows = 16;  // feature rows of one workgroup of dfa_sum_rows; divides kRangeRows
+constexpr int kSumUnroll = 4;
+
+// One contribution to a feature row: element (pt-camera pair and scale) index of
+// its weights inside the batch entry, and its bilinear weight.
+struct Contribution {
+  uint32_t index;  // ((anchor * pts + pt) * cams + cam) * scales + scale
+  float w;
+};
+
+// The active (anchor, pt) pairs of a (batch entry, camera): workgroup
+// b * cams + cam appends {x, y, pair} to its run of anchors * pts slots of
+// `list` and writes their number. Workgroup 0 clears the contribution cursor.
+__global__ void __launch_bounds__(kListBlock)
+    dfa_list_active(const float *__restrict__ loc, float4 *__restrict__ list,
+                    uint32_t *__restrict__ list_n, uint32_t *__restrict__ cursor, Dims d) {
+  __shared__ uint32_t n_list;
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int cam = static_cast<int>(blockIdx.x) % d.cams, b = static_cast<int>(blockIdx.x) / d.cams;
+  if (tid == 0) n_list = 0u;
+  if (blockIdx.x == 0 && tid == 0) *cursor = 0u;
+  __syncthreads();
+  const int pairs = d.anchors * d.pts;
+  const float *src = loc + (static_cast<size_t>(b) * pairs * d.cams + cam) * 2;
+  float4 *dst = list + static_cast<size_t>(blockIdx.x) * pairs;
+  constexpr int kUnroll = 4;
+  for (int p0 = 0; p0 < pairs; p0 += kUnroll * kListBlock) {
+    float x[kUnroll], y[kUnroll];
+#pragma unroll
+    for (int j = 0; j < kUnroll; ++j) {
+      const int p = min(p0 + j * kListBlock + tid, pairs - 1);
+      x[j] = src[static_cast<size_t>(p) * d.cams * 2];
+      y[j] = src[static_cast<size_t>(p) * d.cams * 2 + 1];
+    }
+#pragma unroll
+    for (int j = 0; j < kUnroll; ++j) {
+      const int p = p0 + j * kListBlock + tid;
+      const bool act = p < pairs && active(x[j], y[j]);
+      const uint64_t m = __ballot(act);
+      uint32_t base = 0;
+      if (lane == 0 && m != 0) base = atomicAdd(&n_list, static_cast<uint32_t>(__popcll(m)));
+      base = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(base)));
+      if (act) {
+        dst[base + __popcll(m & ((uint64_t{1} << lane) - 1))] =
+            make_float4(x[j], y[j], __int_as_float(p), 0.0f);
+      }
+    }
+  }
+  __syncthreads();
+  if (tid == 0) list_n[blockIdx.x] = n_list;
+}
+
+// Contributions of kRangeRows feature rows of one batch entry, sorted by row.
+// The workgroup walks the active pairs of the cameras whose maps meet its rows
+// twice: counting per row in LDS, then, with the counts scanned and its run of
+// `contrib` reserved, storing. rows[b * feat + r] = the row's [start, end) in
+// `contrib`; consecutive rows of a range are consecutive there. Maps may
+// overlap: a row lists the contributions of all of them.
+__global__ void __launch_bounds__(kRangeBlock)
+    dfa_list_rows(const int32_t *__restrict__ shape, const int32_t *__restrict__ start,
+                  const float4 *__restrict__ list, const uint32_t *__restrict__ list_n,
+                  uint32_t *__restrict__ cursor, uint2 *__restrict__ rows,
+                  Contribution *__restrict__ contrib, Dims d, int ranges) {
+  constexpr int kWaves = kRangeBlock / kWave;
+  constexpr int kPer = kRangeRows / kRangeBlock;  // rows scanned by a thread
+  __shared__ View views[kMaxViews];
+  __shared__ uint32_t count[kRangeRows];
+  __shared__ uint32_t wave_total[kWaves];
+  __shared__ uint32_t run_base;
+  stage_views(views, shape, start, d);
+  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  const int lb = msda::xcd_logical_block(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+  const int b = lb / ranges, r0 = (lb % ranges) * kRangeRows;
+  const int n_rows = min(kRangeRows, d.feat - r0);
+  for (int i = tid; i < kRangeRows; i += kRangeBlock) count[i] = 0u;
+  __syncthreads();
+  const int pairs = d.anchors * d.pts;
+  // f(row of the range, pair, camera, scale, bilinear weight) for every corner
+  auto each_corner = [&](auto &&f) {
+    for (int cam = 0; cam < d.cams; ++cam) {
+      const int bc = b * d.cams + cam;
+      const int n = static_cast<int>(list_n[bc]);
+      for (int s = 0; s < d.scales; ++s) {
+        const View v = views[cam * d.scales + s];
+        if (v.start + v.h * v.w <= r0 || v.start >= r0 + n_rows) continue;  // uniform
+        for (int i = tid; i < n; i += kRangeBlock) {
+          const float4 e = list[static_cast<size_t>(bc) * pairs + i];
+          const Tap tp = make_tap(e.x, e.y, v);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const int r = v.start + tp.cell[k] - r0;
+            if (tp.cell[k] >= 0 && r >= 0 && r < n_rows) {
+              f(r, __float_as_int(e.z), cam, s, tp.w[k]);
+            }
+          }
+        }
+      }
+    }
+  };
+  each_corner([&](int r, int, int, int, float) { atomicAdd(&count[r], 1u); });
+  __syncthreads();
+  uint32_t c[kPer], sum = 0u;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    c[j] = count[tid * kPer + j];
+    sum += c[j];
+  }
+  const uint32_t upto = msda::wave_inclusive_sum(sum);
+  if (lane == kWave - 1) wave_total[wave] = upto;
+  __syncthreads();
+  if (tid == 0) {
+    uint32_t total = 0u;
+    for (int w = 0; w < kWaves; ++w) total += wave_total[w];
+    run_base = total > 0u ? atomicAdd(cursor, total) : 0u;
+  }
+  __syncthreads();
+  uint32_t at = run_base + upto - sum;
+  for (int w = 0; w < wave; ++w) at += wave_total[w];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int r = tid * kPer + j;
+    count[r] = at;  // the row's write cursor
+    if (r < n_rows) rows[static_cast<size_t>(b) * d.feat + r0 + r] = make_uint2(at, at + c[j]);
+    at += c[j];
+  }
+  __syncthreads();
+  each_corner([&](int r, int pair, int cam, int s, float w) {
+    const uint32_t slot = atomicAdd(&count[r], 1u);
+    contrib[slot] = {static_cast<uint32_t>((pair * d.cams + cam) * d.scales + s), w};
+  });
+}
+
+// grad_feat of kSumRows consecutive feature rows per workgroup, every row
+// written (zero without contributions). The rows' contributions, contiguous,
+// are split evenly over the four wavefronts, so a row that takes many is
+// shared; a wavefront's sum of a row that an earlier wavefront began goes
+// through LDS to the wavefront that began it. A lane holds NT channels
+// (Lanes); a wavefront requests kSumUnroll grad_out rows and weights at a
+// time. Rows are taken from the last to the first: the small maps, whose rows
+// take many contributions, end each camera's rows and so start early.
+template <int NT>
+__global__ void __launch_bounds__(kBlock)
+    dfa_sum_rows(const float *__restrict__ weights, const float *__restrict__ grad_out,
+                 const uint2 *__restrict__ rows, const Contribution *__restrict__ contrib,
+                 float *__restrict__ grad_feat, Dims d, int blocks_per_entry) {
+  using L = Lanes<NT>;
+  constexpr int C = NT * kWave, kWaves = kBlock / kWave;
+  __shared__ double head[kWaves][NT][kWave];  // sum of the row begun by an earlier wavefront
+  __shared__ int through[kWaves];             // ... which goes on past this wavefront's share
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+  const int lb = static_cast<int>(gridDim.x) - 1 -
+                 msda::xcd_logical_block(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+  const int b = lb / blocks_per_entry, r0 = (lb % blocks_per_entry) * kSumRows;
+  const int n = min(kSumRows, d.feat - r0);
+  const size_t row0 = static_cast<size_t>(b) * d.feat + r0;
+  const uint2 mine = rows[row0 + min(lane, n - 1)];  // lane i: row i's contributions
+  auto lane_of = [](uint32_t v, int l) {
+    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), l));
+  };
+  const uint32_t first = lane_of(mine.x, 0), last = lane_of(mine.y, n - 1);
+  const uint32_t share = (last - first + kWaves - 1) / kWaves;
+  const uint32_t e0 = min(first + wave * share, last), e1 = min(e0 + share, last);
+
+  const int cpg = C / d.groups;
+  int grp[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) grp[t] = L::channel(lane, t) / cpg;
+  // grad_out rows and weights at scalar offsets inside the batch entry (the
+  // host keeps both under 2 GiB): no address arithmetic in vector registers
+  const uint32_t per_anchor = static_cast<uint32_t>(d.pts * d.cams * d.scales);
+  const size_t entry_weights = static_cast<size_t>(d.anchors) * per_anchor * d.groups;
+  const __amdgpu_buffer_rsrc_t go =
+      msda::make_rsrc(grad_out + static_cast<size_t>(b) * d.anchors * C,
+                      static_cast<uint32_t>(d.anchors) * (C * 4u));
+  const __amdgpu_buffer_rsrc_t wt =
+      msda::make_rsrc(weights + b * entry_weights, static_cast<uint32_t>(entry_weights * 4));
+
+  double acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = 0.0;
+  auto write = [&](int r) {
+    float o[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) o[t] = static_cast<float>(acc[t]);
+    L::store_nt(grad_feat + (row0 + r) * C, lane, o);
+  };
+  // the row of contribution e0: the first one that ends past it
+  int r = __builtin_popcountll(__ballot(lane < n && mine.y <= e0));
+  uint32_t end = 0u;
+  bool is_head = false;  // row r began in an earlier wavefront's share
+  if (e0 < e1) {
+    end = lane_of(mine.y, r);
+    is_head = lane_of(mine.x, r) < e0;
+  }
+  auto finish_row = [&](bool open) {  // row r's sum over this share is complete
+    if (is_head) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) head[wave][t][lane] = acc[t];
+      if (lane == 0) through[wave] = open ? 1 : 0;
+    } else {
+      write(r);
+    }
+  };
+  for (uint32_t base = e0; base < e1; base += kWave) {
+    const int m = static_cast<int>(min(e1 - base, static_cast<uint32_t>(kWave)));
+    const Contribution ct = contrib[base + min(lane, m - 1)];
+    const uint32_t anchor = ct.index / per_anchor;
+    for (int j0 = 0; j0 < m; j0 += kSumUnroll) {
+      float g[kSumUnroll][NT], wv[kSumUnroll][L::kGroups];
+#pragma unroll
+      for (int u = 0; u < kSumUnroll; ++u) {
+        const int l = min(j0 + u, m - 1);
+        L::gather(go, 0u, lane, g[u], lane_of(anchor, l) * (C * 4u));
+        const uint32_t at = lane_of(ct.index, l) * static_cast<uint32_t>(d.groups) * 4u;
+#pragma unroll
+        for (int t = 0; t < L::kGroups; ++t) wv[u][t] = buffer_load4(wt, grp[t] * 4u, at);
+      }
+#pragma unroll
+      for (int u = 0; u < kSumUnroll; ++u) {
+        if (j0 + u < m) {  // uniform
+          while (base + j0 + u >= end) {  // on to the next row, past empty ones
+            if (lane_of(mine.x, r) != end) finish_row(false);
+            is_head = false;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[t] = 0.0;
+            end = lane_of(mine.y, ++r);
+          }
+          const double w = __uint_as_float(lane_of(__float_as_uint(ct.w), j0 + u));
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            acc[t] = fma(w, static_cast<double>(g[u][t] * wv[u][L::kPacked ? 0 : t]), acc[t]);
+          }
+        }
+      }
+    }
+  }
+  const bool open = e0 < e1 && end > e1;  // row r goes on in the next wavefront's share
+  if (e0 < e1 && (is_head || !open)) finish_row(open);
+  __syncthreads();
+  if (open && !is_head) {
+    for (int w = wave + 1; w < kWaves; ++w) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] += head[w][t][lane];
+      if (through[w] == 0) break;
+    }
+    write(r);
+  }
+  const uint64_t empty = __ballot(lane < n && mine.x == mine.y);
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = 0.0;
+  for (int i = wave; i < n; i += kWaves) {
+    if ((empty >> i) & 1) write(i);
+  }
+}
+
+__global__ void __launch_bounds__(kBlock) dfa_zero(float *__restrict__ p, int64_t n) {
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    p[i] = 0.0f;
   }
 }
 

@@ -6,7 +6,8 @@ Mirrors the reference operator module
 ``reference``, the SparseDrive-compatible ``deformable_aggregation_function``,
 the PyTorch ``deformable_aggregation_reference`` and the ``feature_maps_format``
 helper. The native backend calls the HIP kernels of ``libmuspace_msda.so``
-(``deformable_aggregation_{forward,backward}_opt``, include/muspace_dfa.h).
+(``deformable_aggregation_forward_opt``, ``deformable_aggregation_backward_ws``,
+include/muspace_dfa.h).
 
 Semantics (reference ops:88-158 and the kernels it mirrors): for every
 (batch b, anchor a), over sample points p and cameras c whose normalised
@@ -148,11 +149,11 @@ class _NativeDeformableAggregationFunction(torch.autograd.Function):
         mc_ms_feat, spatial_shape, scale_start_index, sampling_location, weights = (
             ctx.saved_tensors
         )
-        # feature gradients accumulate (atomics); the other two are written in full
-        grad_mc_ms_feat = torch.zeros_like(mc_ms_feat)
+        # the kernels write all three in full
+        grad_mc_ms_feat = torch.empty_like(mc_ms_feat)
         grad_sampling_location = torch.empty_like(sampling_location)
         grad_weights = torch.empty_like(weights)
-        ext.deformable_aggregation_backward_opt(
+        ext.deformable_aggregation_backward(
             mc_ms_feat, spatial_shape, scale_start_index, sampling_location, weights,
             grad_output.float().contiguous(), grad_mc_ms_feat, grad_sampling_location,
             grad_weights,

@@ -137,6 +137,10 @@ _EXPORTS: dict[str, tuple[Any, list[Any]]] = {
     "deformable_aggregation_forward_base": (_c_int, [_c_ptr] * 6 + [_c_int64] * 8 + [_c_ptr]),
     "deformable_aggregation_backward_opt": (_c_int, [_c_ptr] * 9 + [_c_int64] * 8 + [_c_ptr]),
     "deformable_aggregation_backward_base": (_c_int, [_c_ptr] * 9 + [_c_int64] * 8 + [_c_ptr]),
+    "deformable_aggregation_backward_workspace_size": (ctypes.c_size_t, [_c_int64] * 8),
+    "deformable_aggregation_backward_ws": (
+        _c_int, [_c_ptr] * 9 + [_c_int64] * 8 + [_c_ptr, ctypes.c_size_t, _c_ptr]
+    ),
 }
 
 
@@ -233,6 +237,7 @@ class NativeLibrary:
             "deformable_aggregation_forward_base": self.deformable_aggregation_forward_base,
             "deformable_aggregation_backward_opt": self.deformable_aggregation_backward_opt,
             "deformable_aggregation_backward_base": self.deformable_aggregation_backward_base,
+            "deformable_aggregation_backward": self.deformable_aggregation_backward,
             "ms_deform_attn_scatter_div_grad": self.ms_deform_attn_scatter_div_grad,
             "add_one": self.add_one,
         }
@@ -852,7 +857,7 @@ class NativeLibrary:
 
     def _dfa_backward(self, name, mc_ms_feat, spatial_shape, scale_start_index,
                       sampling_location, weights, grad_output, grad_mc_ms_feat,
-                      grad_sampling_location, grad_weights) -> None:
+                      grad_sampling_location, grad_weights, with_workspace=False) -> None:
         import torch
 
         dims = self._dfa_dims(mc_ms_feat, spatial_shape, scale_start_index, sampling_location,
@@ -866,11 +871,17 @@ class NativeLibrary:
             _check(tensor, label, (torch.float32,))
             _check_shape(tensor, label, like)
         with torch.cuda.device(mc_ms_feat.device):
+            scratch = ()
+            if with_workspace:
+                nbytes = self._raw["deformable_aggregation_backward_workspace_size"](*dims)
+                workspace = torch.empty(max(nbytes, 1), dtype=torch.uint8,
+                                        device=mc_ms_feat.device)
+                scratch = (workspace.data_ptr(), nbytes)
             rc = self._raw[name](
                 mc_ms_feat.data_ptr(), spatial_shape.data_ptr(), scale_start_index.data_ptr(),
                 sampling_location.data_ptr(), weights.data_ptr(), grad_output.data_ptr(),
                 grad_mc_ms_feat.data_ptr(), grad_sampling_location.data_ptr(),
-                grad_weights.data_ptr(), *dims, self._stream(mc_ms_feat),
+                grad_weights.data_ptr(), *dims, *scratch, self._stream(mc_ms_feat),
             )
         self._raise_on(rc, name)
 
@@ -894,6 +905,17 @@ class NativeLibrary:
         self._dfa_backward("deformable_aggregation_backward_opt", mc_ms_feat, spatial_shape,
                            scale_start_index, sampling_location, weights, grad_output,
                            grad_mc_ms_feat, grad_sampling_location, grad_weights)
+
+    def deformable_aggregation_backward(self, mc_ms_feat, spatial_shape, scale_start_index,
+                                        sampling_location, weights, grad_output,
+                                        grad_mc_ms_feat, grad_sampling_location,
+                                        grad_weights) -> None:
+        """All three gradients overwritten (none needs zero-filling); the
+        scratch comes from torch's caching allocator."""
+        self._dfa_backward("deformable_aggregation_backward_ws", mc_ms_feat, spatial_shape,
+                           scale_start_index, sampling_location, weights, grad_output,
+                           grad_mc_ms_feat, grad_sampling_location, grad_weights,
+                           with_workspace=True)
 
     def deformable_aggregation_backward_base(self, mc_ms_feat, spatial_shape,
                                              scale_start_index, sampling_location, weights,

@@ -1,0 +1,159 @@
+"""Feature gradients of deformable aggregation summed by owner (the operator's
+backward, deformable_aggregation_backward_ws): where its counting sort and its
+split of a row among wavefronts can go wrong, against the float64 oracle.
+
+The sums are float64 over exact products of float32 factors, rounded once; the
+factors (a bilinear weight, grad_output times a weight) carry one or two
+float32 roundings each, so an element is within 4 * 2^-24 of the sum of its
+contributions' magnitudes. Locations sit on a 1/4096 grid, where the float32
+cell coordinates are exact.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from conftest import gpu_available
+from muspace_amd.runtime.native import load_native_module
+from oracle import dfa_torch
+from test_dfa_oracle import random_case
+
+
+
+def gpu(test):
+    return pytest.mark.gpu(pytest.mark.skipif(not gpu_available(), reason="AMD GPU required")(test))
+
+
+DEV = "cuda"
+
+
+def _case(seed, shapes, channels, groups, anchors, batch=2, pts=3, cams=3):
+    case = list(random_case(seed, batch=batch, anchors=anchors, pts=pts, cams=cams, shapes=shapes,
+                            channels=channels, groups=groups, dtype=torch.float32))
+    case[3].copy_(torch.round(case[3] * 4096) / 4096)
+    return case
+
+
+def _backward(case, grad_out, name="deformable_aggregation_backward"):
+    mc, spatial, start, loc, weights = [t.to(DEV) for t in case]
+    poison = float("nan") if name == "deformable_aggregation_backward" else 0.0
+    grads = [torch.full_like(t, poison) for t in (mc, loc, weights)]
+    getattr(load_native_module(), name)(mc, spatial, start, loc, weights, grad_out.to(DEV), *grads)
+    return [g.cpu() for g in grads]
+
+
+def _oracle(case, grad_out):
+    ref = [t.double().requires_grad_(True) if t.is_floating_point() else t for t in case]
+    (dfa_torch.aggregate_batched(*ref) * grad_out.double()).sum().backward()
+    return [ref[i].grad for i in (0, 3, 4)]
+
+
+def _check(case, grad_out):
+    actual, expected = _backward(case, grad_out), _oracle(case, grad_out)
+    magnitude = _oracle([case[0], *case[1:4], case[4].abs()], grad_out.abs())[0]
+    assert ((actual[0].double() - expected[0]).abs() <= 4 * 2.0**-24 * magnitude + 1e-30).all()
+    torch.testing.assert_close(actual[1].double(), expected[1], rtol=1e-4, atol=1e-3)
+    torch.testing.assert_close(actual[2].double(), expected[2], rtol=1e-4, atol=1e-4)
+
+
+# one to four channel slots; feature rows: fewer than a workgroup's 16, not a
+# multiple of 16, one range of 2048 and a part of the next, several ranges
+@pytest.mark.parametrize("channels,groups", [(64, 8), (128, 4), (192, 3), (256, 8), (256, 1)])
+@pytest.mark.parametrize("shapes", [((2, 2),), ((7, 9), (3, 5)), ((25, 28), (2, 2), (1, 1)),
+                                    ((64, 44), (32, 22), (16, 11))])
+@gpu
+def test_row_ranges_and_channel_layouts(channels, groups, shapes):
+    case = _case(31, shapes, channels, groups, anchors=40)
+    _check(case, torch.randn(2, 40, channels, generator=torch.Generator().manual_seed(32)))
+
+
+@gpu
+@pytest.mark.parametrize("where", [(0.5, 0.5), (0.02, 0.02), (0.99, 0.5)])
+def test_rows_shared_by_wavefronts(where):
+    """Every point of every anchor at one place: a few rows take thousands of
+    contributions, over all four wavefronts of their workgroup."""
+    case = _case(33, ((9, 13), (4, 6), (1, 1)), 256, 8, anchors=333)
+    case[3][...] = torch.tensor([round(w * 4096) / 4096 for w in where])
+    _check(case, torch.randn(2, 333, 256, generator=torch.Generator().manual_seed(34)))
+
+
+@gpu
+def test_overlapping_and_out_of_range_maps():
+    """Maps that share rows list all their contributions there; a map past
+    num_feat adds nothing; rows of no map are zero."""
+    case = _case(35, ((6, 8), (4, 5)), 128, 8, anchors=50)
+    start = case[2]
+    start[0, 1] = start[0, 0] + 7  # camera 0: the second map inside the first
+    start[1, 0] = case[0].shape[1] - 10  # camera 1: its first map would leave the features
+    grad_out = torch.randn(2, 50, 128, generator=torch.Generator().manual_seed(36))
+    actual, base = (_backward(case, grad_out, f"deformable_aggregation_backward{suffix}")
+                    for suffix in ("", "_base"))
+    torch.testing.assert_close(actual[0], base[0], rtol=1e-5, atol=1e-5)
+    torch.testing.assert_close(actual[1], base[1], rtol=1e-4, atol=1e-3)
+    torch.testing.assert_close(actual[2], base[2], rtol=1e-4, atol=1e-4)
+
+
+@gpu
+def test_non_finite_gradients_and_weights():
+    """inf and NaN reach the elements that the base kernels give them."""
+    case = _case(37, ((9, 13), (4, 6)), 256, 8, anchors=60)
+    case[4][0, 3, 1, 2, 0, 5] = float("inf")
+    grad_out = torch.randn(2, 60, 256, generator=torch.Generator().manual_seed(38))
+    grad_out[0, 5, 40] = float("inf")
+    grad_out[1, 9, 3] = float("nan")
+    actual, base = (_backward(case, grad_out, f"deformable_aggregation_backward{suffix}")
+                    for suffix in ("", "_base"))
+    assert not torch.isfinite(base[0]).all()
+    for a, b, atol in zip(actual, base, (1e-4, 1e-3, 1e-4)):
+        torch.testing.assert_close(a, b, rtol=1e-4, atol=atol, equal_nan=True)
+
+
+@gpu
+def test_no_active_point():
+    """Nothing sampled: every gradient is written, as zero."""
+    case = _case(39, ((7, 9),), 64, 8, anchors=20)
+    case[3][...] = 2.0
+    grad_out = torch.ones(2, 20, 64)
+    assert all((g == 0).all() for g in _backward(case, grad_out))
+
+
+@gpu
+def test_captured_backward_replays():
+    """A graph of the backward, replayed on changed inputs, equals the eager call."""
+    case = [t.to(DEV) for t in _case(41, ((9, 13), (4, 6)), 256, 8, anchors=60)]
+    grad_out = torch.randn(2, 60, 256, generator=torch.Generator().manual_seed(42)).to(DEV)
+    lib = load_native_module()
+    grads = [torch.empty_like(case[i]) for i in (0, 3, 4)]
+    lib.deformable_aggregation_backward(*case, grad_out, *grads)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        lib.deformable_aggregation_backward(*case, grad_out, *grads)
+    for step in range(3):
+        grad_out.mul_(-0.5)
+        case[3].copy_((case[3] + 0.125 * step) % 1.0)
+        eager = [torch.empty_like(g) for g in grads]
+        lib.deformable_aggregation_backward(*case, grad_out, *eager)
+        for g in grads:
+            g.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        for g, e in zip(grads, eager):
+            torch.testing.assert_close(g, e, rtol=1e-6, atol=1e-6)
+
+
+def test_workspace_size_and_validation(native_lib):
+    size = native_lib.raw("deformable_aggregation_backward_workspace_size")
+    dims = [2, 3, 500, 256, 2, 40, 4, 8]  # batch, cams, feat, embeds, scales, anchors, pts, groups
+    need = 2 * 3 * 160 * 16 + 2 * 500 * 8 + 4 * 2 * 160 * 3 * 2 * 8
+    assert need <= size(*dims) <= need + 5 * 256
+    assert size(2, 3, 500, 96, 2, 40, 4, 8) == 0  # no row kernel for 96 channels
+    assert size(2, 3, 500, 256, 2, 0, 4, 8) == 0  # nothing sampled
+    assert size(2, 3, 500, 256, 2, 40, 4, 9) == 0  # invalid
+    assert size(64, 6, 2000, 256, 4, 1 << 20, 8, 8) == 0  # past 32-bit offsets
+    fn = native_lib.raw("deformable_aggregation_backward_ws")
+    assert fn(*[1] * 5, None, *[1] * 3, *dims, None, 0, None) == 1  # grad_output NULL
+    assert "null tensor pointer" in native_lib.last_error()
+    assert fn(*[1] * 9, *dims[:7], 9, None, 0, None) == 1
+    assert "num_groups must be in [1, 8]" in native_lib.last_error()
