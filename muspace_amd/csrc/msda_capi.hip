@@ -144,12 +144,24 @@ Launch plan_rows(const msda::Shape &s, int kq, int max_ns, bool forward) {
   if (L.ns > kq) L.ns = kq;  // the forward computes one tap per lane: ng * ns <= 64
   if (L.ns > max_ns) L.ns = max_ns;
   L.plan.gu_log2 = log2_int(gu);
-  L.plan.iters = 8;  // units per lane group: the next unit's geometry loads overlap the gathers
   const int64_t units_per_wave_iter = ng / gu;
   const int64_t wave_iters = (s.units + units_per_wave_iter - 1) / units_per_wave_iter;
-  const int64_t waves = (wave_iters + L.plan.iters - 1) / L.plan.iters;
   const int64_t per_block = msda::kBlock / msda::kWave;
-  L.blocks = static_cast<int>((waves + per_block - 1) / per_block);
+  // units per lane group: 8 (the next unit's geometry loads overlap the
+  // gathers, and a block's prologue is shared by more units), fewer where 8
+  // would leave the 256 CUs short of two blocks each. Measured at 8 and as
+  // chosen: 1000 queries x 8 heads x 16 samples fp32 (63 -> 500 blocks) 15.1 ->
+  // 7.5 us, 300 queries fp16 14.3 -> 5.4 us, the fused binning forward at 2 x
+  // 900 queries 31.2 -> 17.5 us (its bin_count 14.1 -> 9.1 us). Where 8 fills
+  // the chip already, fewer is slower: 2 x 22223 queries 196 us at 8, 210 at 4,
+  // 252 at 2.
+  L.plan.iters = 8;
+  do {
+    const int64_t waves = (wave_iters + L.plan.iters - 1) / L.plan.iters;
+    L.blocks = static_cast<int>((waves + per_block - 1) / per_block);
+    if (L.blocks >= 512 || L.plan.iters == 1) break;
+    L.plan.iters /= 2;
+  } while (true);
   return L;
 }
 
