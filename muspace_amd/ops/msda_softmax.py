@@ -25,7 +25,6 @@ the probabilities. Gradients and dtypes follow ``multi_scale_deformable_attn``.
 
 from __future__ import annotations
 
-import weakref
 
 import torch
 
@@ -38,6 +37,7 @@ from ..runtime.kernel_dispatch import (
 )
 from ..runtime.native import native_error
 from .multi_scale_deformable_attn import (
+    Reservation,
     _bins_early,
     _native_extension,
     _reserve_early_buffers,
@@ -70,9 +70,9 @@ def _binning_buffers(ext, value, sampling, logits):
     except BaseException:
         release()  # nothing was allocated: the reservation goes back now
         raise
-    # from here on the workspace's finalizer returns the reservation, also
-    # when an allocation below raises and drops the workspace
-    weakref.finalize(workspace, release)
+    # from here on the workspace's end returns the reservation, also when an
+    # allocation below raises and drops the workspace
+    workspace.reservation = Reservation(release)
     device = value.device
     grads = (
         torch.empty(value.shape, dtype=torch.float32, device=device),

@@ -33,7 +33,6 @@ from __future__ import annotations
 import os
 import threading
 import warnings
-import weakref
 
 import torch
 import torch.nn.functional as F
@@ -192,6 +191,19 @@ class BinningBudget:
 binning_budget = BinningBudget()
 
 
+class Reservation:
+    """Calls ``release`` when dropped: held as an attribute of the tensor whose
+    bytes it stands for."""
+
+    __slots__ = ("_release",)
+
+    def __init__(self, release) -> None:
+        self._release = release
+
+    def __del__(self) -> None:
+        self._release()
+
+
 def _device_index(device: torch.device) -> int:
     return device.index if device.index is not None else torch.cuda.current_device()
 
@@ -208,7 +220,8 @@ def _reserve_early_buffers(workspace_bytes: int, *like: torch.Tensor):
 
 
 def _early_binning_enabled() -> bool:
-    return os.environ.get(EARLY_BINNING_ENV, "1").strip().lower() not in {"0", "false", "no", "off"}
+    raw = os.environ.get(EARLY_BINNING_ENV)
+    return raw is None or raw.strip().lower() not in {"0", "false", "no", "off"}
 
 
 def _bins_early(*tensors: torch.Tensor) -> bool:
@@ -234,9 +247,9 @@ def _binning_buffers(ext, value, sampling, attn):
     except BaseException:
         release()  # nothing was allocated: the reservation goes back now
         raise
-    # from here on the workspace's finalizer returns the reservation, also
-    # when an allocation below raises and drops the workspace
-    weakref.finalize(workspace, release)
+    # from here on the workspace's end returns the reservation, also when an
+    # allocation below raises and drops the workspace
+    workspace.reservation = Reservation(release)
     device = value.device
     grads = (
         torch.empty(value.shape, dtype=torch.float32, device=device),

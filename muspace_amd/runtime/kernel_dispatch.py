@@ -34,6 +34,7 @@ SelectedBackend = Literal["hip", "reference", "error"]
 
 NATIVE_BACKEND = "hip"
 NATIVE_ALIASES = frozenset({"hip", "musa"})
+_BACKENDS = NATIVE_ALIASES | {"auto", "reference"}
 MAX_REPORTS = 4096
 LOG_ENV = "MUSPACE_DISPATCH_LOG"
 AUTO_FALLBACK_ENV = "MUSPACE_AUTO_FALLBACK"
@@ -69,7 +70,8 @@ _dispatch_reports: deque[DispatchReport] = deque(maxlen=MAX_REPORTS)
 
 
 def _env_flag(name: str) -> bool:
-    return os.environ.get(name, "").strip().lower() in {"1", "true", "yes", "on"}
+    raw = os.environ.get(name)
+    return raw is not None and raw.strip().lower() in {"1", "true", "yes", "on"}
 
 
 def _log_enabled() -> bool:
@@ -111,9 +113,9 @@ def explain_dispatch(
     backend: str = "auto",
     native_available: bool = True,
 ) -> DispatchDecision:
-    if backend not in {"auto", "reference"} | NATIVE_ALIASES:
-        return DispatchDecision("error", value.device.type, f"unknown backend: {backend}")
     device = value.device.type
+    if backend not in _BACKENDS:
+        return DispatchDecision("error", device, f"unknown backend: {backend}")
     if backend == "reference":
         return DispatchDecision("reference", device, "reference backend requested")
 

@@ -24,6 +24,8 @@ from importlib.resources import files
 from pathlib import Path
 from typing import Any, Callable
 
+import torch
+
 LIBRARY_RELPATH = "native/libmuspace_msda.so"
 ABI_VERSION = 6
 
@@ -152,12 +154,12 @@ def library_path() -> Path:
     return Path(files("muspace_amd").joinpath(LIBRARY_RELPATH))
 
 
-def _dtype_code(dtype) -> int:
-    import torch
+_DTYPE_CODES = {torch.float32: DTYPE_F32, torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16}
 
-    codes = {torch.float32: DTYPE_F32, torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16}
+
+def _dtype_code(dtype) -> int:
     try:
-        return codes[dtype]
+        return _DTYPE_CODES[dtype]
     except KeyError:
         raise RuntimeError(f"unsupported dtype {dtype}") from None
 
@@ -189,6 +191,53 @@ def _check_shape(tensor, name: str, shape: tuple[int, ...]) -> None:
         raise RuntimeError(f"{name} must have shape {list(shape)}, got {list(tensor.shape)}")
 
 
+def _all_on(device, *tensors) -> bool:
+    """Every tensor a contiguous one in GPU memory, on ``device``."""
+    for tensor in tensors:
+        if (tensor is None or not _is_device_tensor(tensor) or tensor.device != device
+                or not tensor.is_contiguous()):
+            return False
+    return True
+
+
+def _forward_dims(value, spatial_shapes, level_start_index, sampling_locations,
+                  attention_weights, output) -> tuple[int, ...] | None:
+    """The dims of a forward whose tensors pass every check of
+    :meth:`NativeLibrary.check_forward`, else None."""
+    if value is None or sampling_locations is None or not _all_on(
+            value.device, value, spatial_shapes, level_start_index, sampling_locations,
+            attention_weights):
+        return None
+    dtype, geometry = value.dtype, sampling_locations.dtype
+    if (dtype not in _DTYPE_CODES or (geometry != torch.float32 and geometry != dtype)
+            or attention_weights.dtype != geometry or spatial_shapes.dtype != torch.int64
+            or level_start_index.dtype != torch.int64 or value.dim() != 4
+            or sampling_locations.dim() != 6 or spatial_shapes.dim() != 2):
+        return None
+    batch, spatial, heads, channels = value.shape
+    levels = spatial_shapes.shape[0]
+    queries, points = sampling_locations.shape[1], sampling_locations.shape[4]
+    if (spatial_shapes.shape != (levels, 2) or level_start_index.shape != (levels,)
+            or sampling_locations.shape != (batch, queries, heads, levels, points, 2)
+            or attention_weights.shape != (batch, queries, heads, levels, points)):
+        return None
+    if output is not None and (not _all_on(value.device, output) or output.dtype != dtype
+                               or output.shape != (batch, queries, heads * channels)):
+        return None
+    return batch, spatial, heads, channels, levels, queries, points
+
+
+# the raw handle of a device's current stream: torch's own accessor for
+# launchers where there is one (current_stream builds a Stream object per call)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _stream_of(device) -> int:
+    if _raw_stream is not None:
+        return _raw_stream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
+
+
 class NativeLibrary:
     """The loaded library with its exports bound once."""
 
@@ -211,6 +260,8 @@ class NativeLibrary:
                 f"muSPACE native library {path} has ABI version {version}, expected {ABI_VERSION}; "
                 "rebuild it with `python -m muspace_amd.build`"
             )
+        # scratch sizes by device and dims (a plan each, asked for several times a step)
+        self._size = lru_cache(maxsize=1024)(self._workspace_size)
         self._bound: dict[str, Callable[..., Any]] = {
             "check_forward": self.check_forward,
             "check_backward": self.check_backward,
@@ -267,11 +318,18 @@ class NativeLibrary:
         if rc != 0:
             raise RuntimeError(self.last_error() or f"{name} failed with code {rc}")
 
-    @staticmethod
-    def _stream(tensor) -> int:
-        import torch
-
-        return torch.cuda.current_stream(tensor.device).cuda_stream
+    def _launch(self, name: str, device, *args, stream: int | None = None) -> None:
+        """Call export ``name`` with ``args`` and, last, the stream handle
+        (``None``: ``device``'s current stream), with ``device`` current (entered
+        only when it is not)."""
+        if stream is None:
+            stream = _stream_of(device)
+        if device.index == torch.cuda.current_device():
+            rc = self._raw[name](*args, stream)
+        else:
+            with torch.cuda.device(device):
+                rc = self._raw[name](*args, stream)
+        self._raise_on(rc, name)
 
     # ------------------------------------------------------ tensor entry ---
     def ms_deform_attn_forward(
@@ -304,8 +362,11 @@ class NativeLibrary:
         part of the backward has none). Raises RuntimeError; returns
         (batch, spatial, heads, channels, levels, queries, points).
         """
-        import torch
-
+        dims = _forward_dims(value, spatial_shapes, level_start_index, sampling_locations,
+                             attention_weights, output)
+        if dims is not None:
+            return dims
+        # something is wrong: one check at a time, for its message
         _check(value, "value", (torch.float32, torch.float16, torch.bfloat16))
         dev = value.device
         _check(spatial_shapes, "spatial_shapes", (torch.int64,), dev)
@@ -332,15 +393,13 @@ class NativeLibrary:
 
     def check_backward(self, value, spatial_shapes, level_start_index, sampling_locations,
                        attention_weights, grad_output, grad_value, grad_sampling_locations,
-                       grad_attention_weights) -> tuple[int, ...]:
+                       grad_attention_weights, output=None) -> tuple[int, ...]:
         """Validate the backward's tensors (as :meth:`check_forward`, plus
         grad_output in the value's dtype and three float32 gradients of the
         inputs' shapes). ``grad_output`` is None for the binning part, which
         does not read it. Raises RuntimeError; returns the dims."""
-        import torch
-
         dims = self.check_forward(value, spatial_shapes, level_start_index, sampling_locations,
-                                  attention_weights)
+                                  attention_weights, output)
         batch, _, heads, channels, _, queries, _ = dims
         dev = value.device
         if grad_output is not None:
@@ -357,20 +416,17 @@ class NativeLibrary:
 
     def _forward_call(self, name, value, spatial_shapes, level_start_index, sampling_locations,
                       attention_weights, output, im2col_step) -> None:
-        import torch
-
         batch, spatial, heads, channels, levels, queries, points = self.check_forward(
             value, spatial_shapes, level_start_index, sampling_locations, attention_weights,
             output)
-        with torch.cuda.device(value.device):
-            rc = self._raw[name](
-                value.data_ptr(), _dtype_code(value.dtype), spatial_shapes.data_ptr(),
-                level_start_index.data_ptr(), sampling_locations.data_ptr(),
-                attention_weights.data_ptr(), _dtype_code(sampling_locations.dtype),
-                output.data_ptr(), batch, spatial, heads, channels, levels, queries, points,
-                int(im2col_step), self._stream(value),
-            )
-        self._raise_on(rc, name)
+        self._launch(
+            name, value.device,
+            value.data_ptr(), _dtype_code(value.dtype), spatial_shapes.data_ptr(),
+            level_start_index.data_ptr(), sampling_locations.data_ptr(),
+            attention_weights.data_ptr(), _dtype_code(sampling_locations.dtype),
+            output.data_ptr(), batch, spatial, heads, channels, levels, queries, points,
+            int(im2col_step),
+        )
 
     def ms_deform_attn_backward(
         self, value, spatial_shapes, level_start_index, sampling_locations,
@@ -383,18 +439,14 @@ class NativeLibrary:
         The tile-owned kernels' scratch comes from torch's caching allocator
         on the value's device.
         """
-        import torch
-
         self.check_backward(value, spatial_shapes, level_start_index, sampling_locations,
                             attention_weights, grad_output, grad_value, grad_sampling_locations,
                             grad_attention_weights)
-        with torch.cuda.device(value.device):
-            workspace = self.backward_workspace(value, sampling_locations)
-            self._backward_call("ms_deform_attn_backward_ws", value, spatial_shapes,
-                                level_start_index, sampling_locations, attention_weights,
-                                grad_output, grad_value, grad_sampling_locations,
-                                grad_attention_weights, im2col_step, workspace,
-                                self._stream(value))
+        workspace = self.backward_workspace(value, sampling_locations)
+        self._backward_call("ms_deform_attn_backward_ws", value, spatial_shapes,
+                            level_start_index, sampling_locations, attention_weights,
+                            grad_output, grad_value, grad_sampling_locations,
+                            grad_attention_weights, im2col_step, workspace)
 
     def ms_deform_attn_backward_noalloc(
         self, value, spatial_shapes, level_start_index, sampling_locations,
@@ -405,21 +457,18 @@ class NativeLibrary:
         nothing: its scratch is the library's fixed per-GPU array
         (MUSPACE_NOALLOC_SCRATCH_BYTES), the batch processed in passes that fit
         it. Calls that overlap on one GPU race on that array."""
-        import torch
-
         dims = self.check_backward(value, spatial_shapes, level_start_index, sampling_locations,
                                    attention_weights, grad_output, grad_value,
                                    grad_sampling_locations, grad_attention_weights)
-        with torch.cuda.device(value.device):
-            rc = self._raw["ms_deform_attn_backward_noalloc"](
-                value.data_ptr(), _dtype_code(value.dtype), spatial_shapes.data_ptr(),
-                level_start_index.data_ptr(), sampling_locations.data_ptr(),
-                attention_weights.data_ptr(), _dtype_code(sampling_locations.dtype),
-                grad_output.data_ptr(), grad_value.data_ptr(),
-                grad_sampling_locations.data_ptr(), grad_attention_weights.data_ptr(),
-                *dims, int(im2col_step), self._stream(value),
-            )
-        self._raise_on(rc, "ms_deform_attn_backward_noalloc")
+        self._launch(
+            "ms_deform_attn_backward_noalloc", value.device,
+            value.data_ptr(), _dtype_code(value.dtype), spatial_shapes.data_ptr(),
+            level_start_index.data_ptr(), sampling_locations.data_ptr(),
+            attention_weights.data_ptr(), _dtype_code(sampling_locations.dtype),
+            grad_output.data_ptr(), grad_value.data_ptr(),
+            grad_sampling_locations.data_ptr(), grad_attention_weights.data_ptr(),
+            *dims, int(im2col_step),
+        )
 
     def ms_deform_attn_backward_softmax(
         self, value, spatial_shapes, level_start_index, sampling_locations,
@@ -429,31 +478,35 @@ class NativeLibrary:
         """Backward of :meth:`ms_deform_attn_forward_softmax`: the value,
         location and logit gradients, all overwritten. Scratch (the softmax
         probabilities and the binning) comes from torch's caching allocator."""
-        import torch
-
         self.check_backward(value, spatial_shapes, level_start_index, sampling_locations,
                             attention_logits, grad_output, grad_value, grad_sampling_locations,
                             grad_attention_logits)
-        with torch.cuda.device(value.device):
-            workspace = self.backward_softmax_workspace(value, sampling_locations)
-            stream = self._stream(value)
-            for name in ("ms_deform_attn_backward_softmax_bin",
-                         "ms_deform_attn_backward_softmax_rest"):
-                self._backward_call(name, value, spatial_shapes, level_start_index,
-                                    sampling_locations, attention_logits, grad_output,
-                                    grad_value, grad_sampling_locations, grad_attention_logits,
-                                    im2col_step, workspace, stream)
+        workspace = self.backward_softmax_workspace(value, sampling_locations)
+        for name in ("ms_deform_attn_backward_softmax_bin",
+                     "ms_deform_attn_backward_softmax_rest"):
+            self._backward_call(name, value, spatial_shapes, level_start_index,
+                                sampling_locations, attention_logits, grad_output,
+                                grad_value, grad_sampling_locations, grad_attention_logits,
+                                im2col_step, workspace)
 
     def _workspace_bytes(self, value, sampling_locations, softmax: bool) -> int:
         batch, spatial, heads, channels = value.shape
         queries, levels, points = (sampling_locations.shape[1], sampling_locations.shape[3],
                                    sampling_locations.shape[4])
+        types = (_dtype_code(value.dtype),)
         if softmax:
-            return int(self._raw["ms_deform_attn_backward_softmax_workspace_size"](
-                _dtype_code(value.dtype), _dtype_code(sampling_locations.dtype), batch, spatial,
-                heads, channels, levels, queries, points))
-        return int(self._raw["ms_deform_attn_backward_workspace_size"](
-            _dtype_code(value.dtype), batch, spatial, heads, channels, levels, queries, points))
+            types += (_dtype_code(sampling_locations.dtype),)
+        # the plan also depends on the device's compute units
+        return self._size(value.device.index, softmax, *types, batch, spatial, heads, channels,
+                          levels, queries, points)
+
+    def _workspace_size(self, device_index, softmax: bool, *args) -> int:
+        name = ("ms_deform_attn_backward_softmax_workspace_size" if softmax
+                else "ms_deform_attn_backward_workspace_size")
+        if device_index is None or device_index == torch.cuda.current_device():
+            return int(self._raw[name](*args))
+        with torch.cuda.device(device_index):
+            return int(self._raw[name](*args))
 
     def backward_workspace_bytes(self, value, sampling_locations) -> int:
         """Scratch bytes of the tile-owned backward for these shapes (0: the
@@ -486,31 +539,25 @@ class NativeLibrary:
     def backward_workspace(self, value, sampling_locations):
         """Scratch of the tile-owned backward for these shapes (1 byte when the
         shape takes the atomic fallback)."""
-        import torch
-
         nbytes = self._workspace_bytes(value, sampling_locations, softmax=False)
         return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=value.device)
 
     def backward_softmax_workspace(self, value, sampling_locations):
         """Scratch of the softmax backward for these shapes: the probabilities,
         then the tile-owned kernels' scratch when the tile path applies."""
-        import torch
-
         nbytes = self._workspace_bytes(value, sampling_locations, softmax=True)
         return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=value.device)
 
     def _check_split(self, value, spatial_shapes, level_start_index, sampling_locations,
                      attention_weights, grad_output, grad_value, grad_sampling_locations,
-                     grad_attention_weights, workspace, softmax: bool) -> None:
+                     grad_attention_weights, workspace, softmax: bool, output=None) -> None:
         """Checks of one part of a backward split in two (binning, rest): every
         tensor as :meth:`check_backward`, and a workspace of at least the size
         the shapes need, so both parts take the same path (a smaller one
         would make the binning skip the tile path while the rest expects it)."""
-        import torch
-
         self.check_backward(value, spatial_shapes, level_start_index, sampling_locations,
                             attention_weights, grad_output, grad_value, grad_sampling_locations,
-                            grad_attention_weights)
+                            grad_attention_weights, output)
         _check(workspace, "workspace", (torch.uint8,), value.device)
         need = self._workspace_bytes(value, sampling_locations, softmax)
         if workspace.numel() < need:
@@ -519,36 +566,32 @@ class NativeLibrary:
 
     def _backward_call(self, name, value, spatial_shapes, level_start_index, sampling_locations,
                        attention_weights, grad_output, grad_value, grad_sampling_locations,
-                       grad_attention_weights, im2col_step, workspace, stream) -> None:
+                       grad_attention_weights, im2col_step, workspace, stream=None) -> None:
         batch, spatial, heads, channels = value.shape
         levels = spatial_shapes.shape[0]
         queries, points = sampling_locations.shape[1], sampling_locations.shape[4]
-        rc = self._raw[name](
+        self._launch(
+            name, value.device,
             value.data_ptr(), _dtype_code(value.dtype), spatial_shapes.data_ptr(),
             level_start_index.data_ptr(), sampling_locations.data_ptr(),
             attention_weights.data_ptr(), _dtype_code(sampling_locations.dtype),
             None if grad_output is None else grad_output.data_ptr(), grad_value.data_ptr(),
             grad_sampling_locations.data_ptr(), grad_attention_weights.data_ptr(),
             batch, spatial, heads, channels, levels, queries, points,
-            int(im2col_step), workspace.data_ptr(), workspace.numel(), stream,
+            int(im2col_step), workspace.data_ptr(), workspace.numel(), stream=stream,
         )
-        self._raise_on(rc, name)
 
     def _split_part(self, name, softmax, value, spatial_shapes, level_start_index,
                     sampling_locations, attention_weights, grad_output, grad_value,
                     grad_sampling_locations, grad_attention_weights, im2col_step, workspace,
                     stream) -> None:
-        import torch
-
         self._check_split(value, spatial_shapes, level_start_index, sampling_locations,
                           attention_weights, grad_output, grad_value, grad_sampling_locations,
                           grad_attention_weights, workspace, softmax)
-        st = stream if stream is not None else torch.cuda.current_stream(value.device)
-        with torch.cuda.device(value.device):
-            self._backward_call(name, value, spatial_shapes, level_start_index,
-                                sampling_locations, attention_weights, grad_output, grad_value,
-                                grad_sampling_locations, grad_attention_weights, im2col_step,
-                                workspace, st.cuda_stream)
+        self._backward_call(name, value, spatial_shapes, level_start_index, sampling_locations,
+                            attention_weights, grad_output, grad_value,
+                            grad_sampling_locations, grad_attention_weights, im2col_step,
+                            workspace, None if stream is None else stream.cuda_stream)
 
     def ms_deform_attn_backward_bin(
         self, value, spatial_shapes, level_start_index, sampling_locations, attention_weights,
@@ -617,27 +660,21 @@ class NativeLibrary:
     ) -> None:
         """One of the forward + binning calls, every tensor and the workspace
         size checked before the launch."""
-        import torch
-
-        self.check_forward(value, spatial_shapes, level_start_index, sampling_locations,
-                           attention_weights, output)
         self._check_split(value, spatial_shapes, level_start_index, sampling_locations,
                           attention_weights, None, grad_value, grad_sampling_locations,
-                          grad_attention_weights, workspace, softmax)
+                          grad_attention_weights, workspace, softmax, output)
         batch, spatial, heads, channels = value.shape
         levels = spatial_shapes.shape[0]
         queries, points = sampling_locations.shape[1], sampling_locations.shape[4]
-        with torch.cuda.device(value.device):
-            rc = self._raw[name](
-                value.data_ptr(), _dtype_code(value.dtype), spatial_shapes.data_ptr(),
-                level_start_index.data_ptr(), sampling_locations.data_ptr(),
-                attention_weights.data_ptr(), _dtype_code(sampling_locations.dtype),
-                output.data_ptr(), grad_value.data_ptr(), grad_sampling_locations.data_ptr(),
-                grad_attention_weights.data_ptr(), batch, spatial, heads, channels, levels,
-                queries, points, int(im2col_step), workspace.data_ptr(), workspace.numel(),
-                self._stream(value),
-            )
-        self._raise_on(rc, name)
+        self._launch(
+            name, value.device,
+            value.data_ptr(), _dtype_code(value.dtype), spatial_shapes.data_ptr(),
+            level_start_index.data_ptr(), sampling_locations.data_ptr(),
+            attention_weights.data_ptr(), _dtype_code(sampling_locations.dtype),
+            output.data_ptr(), grad_value.data_ptr(), grad_sampling_locations.data_ptr(),
+            grad_attention_weights.data_ptr(), batch, spatial, heads, channels, levels,
+            queries, points, int(im2col_step), workspace.data_ptr(), workspace.numel(),
+        )
 
     def ms_deform_attn_backward_softmax_bin(
         self, value, spatial_shapes, level_start_index, sampling_locations, attention_logits,
@@ -676,8 +713,6 @@ class NativeLibrary:
         the reference's ``ms_deformable_im2col_scatter_div_musa``
         (/root/reference/csrc/ms_deformable_attn/ms_deform_attn_musa.mu:455-505).
         """
-        import torch
-
         half = (torch.float32, torch.float16, torch.bfloat16)
         _check(value, "value", half)
         _check(spatial_shapes, "spatial_shapes", (torch.int64,))
@@ -706,16 +741,15 @@ class NativeLibrary:
         _check_shape(attention_weights, "attention_weights", (rows, max_len, heads, levels, points))
         _check_shape(count, "count", (batch, num_query))
         _check_shape(slots, "slots", (batch, num_query, heads * channels))
-        with torch.cuda.device(value.device):
-            rc = self._raw["ms_deform_attn_forward_scatter_div"](
-                value.data_ptr(), _dtype_code(value.dtype), spatial_shapes.data_ptr(),
-                level_start_index.data_ptr(), sampling_locations.data_ptr(),
-                attention_weights.data_ptr(), _dtype_code(sampling_locations.dtype),
-                index.data_ptr(), count.data_ptr(), slots.data_ptr(), batch, num_cams,
-                int(cam_id), valid_len, spatial, heads, channels, levels, max_len, points,
-                num_query, self._stream(value),
-            )
-        self._raise_on(rc, "ms_deform_attn_forward_scatter_div")
+        self._launch(
+            "ms_deform_attn_forward_scatter_div", value.device,
+            value.data_ptr(), _dtype_code(value.dtype), spatial_shapes.data_ptr(),
+            level_start_index.data_ptr(), sampling_locations.data_ptr(),
+            attention_weights.data_ptr(), _dtype_code(sampling_locations.dtype),
+            index.data_ptr(), count.data_ptr(), slots.data_ptr(), batch, num_cams,
+            int(cam_id), valid_len, spatial, heads, channels, levels, max_len, points,
+            num_query,
+        )
 
     def ms_deform_attn_forward_scatter_div_cams(
         self, value, spatial_shapes, level_start_index, sampling_locations,
@@ -727,8 +761,6 @@ class NativeLibrary:
         with ``index`` the cameras' BEV ids concatenated and ``valid_lens`` (a
         sequence of ints, one per camera) their lengths.
         """
-        import torch
-
         half = (torch.float32, torch.float16, torch.bfloat16)
         _check(value, "value", half)
         _check(spatial_shapes, "spatial_shapes", (torch.int64,))
@@ -762,16 +794,15 @@ class NativeLibrary:
         _check_shape(count, "count", (batch, num_query))
         _check_shape(slots, "slots", (batch, num_query, heads * channels))
         host_lens = (ctypes.c_int64 * num_cams)(*lens)
-        with torch.cuda.device(value.device):
-            rc = self._raw["ms_deform_attn_forward_scatter_div_cams"](
-                value.data_ptr(), _dtype_code(value.dtype), spatial_shapes.data_ptr(),
-                level_start_index.data_ptr(), sampling_locations.data_ptr(),
-                attention_weights.data_ptr(), _dtype_code(sampling_locations.dtype),
-                index.data_ptr(), ctypes.cast(host_lens, ctypes.c_void_p), count.data_ptr(),
-                slots.data_ptr(), batch, num_cams, spatial, heads, channels, levels, max_len,
-                points, num_query, self._stream(value),
-            )
-        self._raise_on(rc, "ms_deform_attn_forward_scatter_div_cams")
+        self._launch(
+            "ms_deform_attn_forward_scatter_div_cams", value.device,
+            value.data_ptr(), _dtype_code(value.dtype), spatial_shapes.data_ptr(),
+            level_start_index.data_ptr(), sampling_locations.data_ptr(),
+            attention_weights.data_ptr(), _dtype_code(sampling_locations.dtype),
+            index.data_ptr(), ctypes.cast(host_lens, ctypes.c_void_p), count.data_ptr(),
+            slots.data_ptr(), batch, num_cams, spatial, heads, channels, levels, max_len,
+            points, num_query,
+        )
 
     def ms_deform_attn_scatter_div_grad(
         self, grad_slots, index, valid_lens, count, grad_output,
@@ -780,8 +811,6 @@ class NativeLibrary:
         num_query, row]``: camera c's row r gets ``grad_slots[b, q] / count[b, q]``
         (q its BEV id in the concatenated ``index``) for r < valid_lens[c], zero
         past it."""
-        import torch
-
         half = (torch.float32, torch.float16, torch.bfloat16)
         _check(grad_slots, "grad_slots", half)
         _check(index, "index", (torch.int64,))
@@ -801,22 +830,19 @@ class NativeLibrary:
         _check_shape(grad_output, "grad_output", (batch * num_cams, max_len, row))
         _check_shape(count, "count", (batch, num_query))
         host_lens = (ctypes.c_int64 * num_cams)(*lens)
-        with torch.cuda.device(grad_slots.device):
-            rc = self._raw["ms_deform_attn_scatter_div_grad"](
-                grad_slots.data_ptr(), _dtype_code(grad_slots.dtype), index.data_ptr(),
-                ctypes.cast(host_lens, ctypes.c_void_p), count.data_ptr(),
-                _dtype_code(count.dtype), grad_output.data_ptr(), batch, num_cams, max_len,
-                num_query, row, self._stream(grad_slots),
-            )
-        self._raise_on(rc, "ms_deform_attn_scatter_div_grad")
+        self._launch(
+            "ms_deform_attn_scatter_div_grad", grad_slots.device,
+            grad_slots.data_ptr(), _dtype_code(grad_slots.dtype), index.data_ptr(),
+            ctypes.cast(host_lens, ctypes.c_void_p), count.data_ptr(),
+            _dtype_code(count.dtype), grad_output.data_ptr(), batch, num_cams, max_len,
+            num_query, row,
+        )
 
     # ------------------------------------------------ deformable aggregation ---
     @staticmethod
     def _dfa_dims(mc_ms_feat, spatial_shape, scale_start_index, sampling_location, weights):
         """Checks of the reference's validate() (deformable_aggregation_musa.mu:669-679)
         and the dims its launchers read (:660-668)."""
-        import torch
-
         _check(mc_ms_feat, "mc_ms_feat", (torch.float32,))
         _check(spatial_shape, "spatial_shape", (torch.int32,))
         _check(scale_start_index, "scale_start_index", (torch.int32,))
@@ -841,25 +867,19 @@ class NativeLibrary:
 
     def _dfa_forward(self, name, mc_ms_feat, spatial_shape, scale_start_index,
                      sampling_location, weights, output) -> None:
-        import torch
-
         dims = self._dfa_dims(mc_ms_feat, spatial_shape, scale_start_index, sampling_location,
                               weights)
         _check(output, "out", (torch.float32,))
         _check_shape(output, "out", (dims[0], dims[5], dims[3]))
-        with torch.cuda.device(mc_ms_feat.device):
-            rc = self._raw[name](
-                mc_ms_feat.data_ptr(), spatial_shape.data_ptr(), scale_start_index.data_ptr(),
-                sampling_location.data_ptr(), weights.data_ptr(), output.data_ptr(), *dims,
-                self._stream(mc_ms_feat),
-            )
-        self._raise_on(rc, name)
+        self._launch(
+            name, mc_ms_feat.device,
+            mc_ms_feat.data_ptr(), spatial_shape.data_ptr(), scale_start_index.data_ptr(),
+            sampling_location.data_ptr(), weights.data_ptr(), output.data_ptr(), *dims,
+        )
 
     def _dfa_backward(self, name, mc_ms_feat, spatial_shape, scale_start_index,
                       sampling_location, weights, grad_output, grad_mc_ms_feat,
                       grad_sampling_location, grad_weights, with_workspace=False) -> None:
-        import torch
-
         dims = self._dfa_dims(mc_ms_feat, spatial_shape, scale_start_index, sampling_location,
                               weights)
         for tensor, label, like in (
@@ -870,20 +890,18 @@ class NativeLibrary:
         ):
             _check(tensor, label, (torch.float32,))
             _check_shape(tensor, label, like)
-        with torch.cuda.device(mc_ms_feat.device):
-            scratch = ()
-            if with_workspace:
-                nbytes = self._raw["deformable_aggregation_backward_workspace_size"](*dims)
-                workspace = torch.empty(max(nbytes, 1), dtype=torch.uint8,
-                                        device=mc_ms_feat.device)
-                scratch = (workspace.data_ptr(), nbytes)
-            rc = self._raw[name](
-                mc_ms_feat.data_ptr(), spatial_shape.data_ptr(), scale_start_index.data_ptr(),
-                sampling_location.data_ptr(), weights.data_ptr(), grad_output.data_ptr(),
-                grad_mc_ms_feat.data_ptr(), grad_sampling_location.data_ptr(),
-                grad_weights.data_ptr(), *dims, *scratch, self._stream(mc_ms_feat),
-            )
-        self._raise_on(rc, name)
+        scratch = ()
+        if with_workspace:
+            nbytes = self._raw["deformable_aggregation_backward_workspace_size"](*dims)
+            workspace = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=mc_ms_feat.device)
+            scratch = (workspace.data_ptr(), nbytes)
+        self._launch(
+            name, mc_ms_feat.device,
+            mc_ms_feat.data_ptr(), spatial_shape.data_ptr(), scale_start_index.data_ptr(),
+            sampling_location.data_ptr(), weights.data_ptr(), grad_output.data_ptr(),
+            grad_mc_ms_feat.data_ptr(), grad_sampling_location.data_ptr(),
+            grad_weights.data_ptr(), *dims, *scratch,
+        )
 
     def deformable_aggregation_forward_opt(self, mc_ms_feat, spatial_shape, scale_start_index,
                                            sampling_location, weights, output) -> None:
@@ -927,17 +945,14 @@ class NativeLibrary:
 
     def add_one(self, value, actual) -> None:
         """Build smoke: actual = value + 1 (float32 device tensors)."""
-        import torch
-
         _check(value, "value", (torch.float32,))
         _check(actual, "actual", (torch.float32,))
         if value.numel() != actual.numel():
             raise RuntimeError("value and actual must have the same number of elements")
-        with torch.cuda.device(value.device):
-            rc = self._raw["add_one"](
-                value.data_ptr(), actual.data_ptr(), value.numel(), self._stream(value)
-            )
-        self._raise_on(rc, "add_one")
+        self._launch(
+            "add_one", value.device,
+            value.data_ptr(), actual.data_ptr(), value.numel(),
+        )
 
 
 @lru_cache(maxsize=1)
