@@ -173,11 +173,12 @@ MUSPACE_API int ms_deform_attn_backward_rest(
 /* ms_deform_attn_forward followed by ms_deform_attn_backward_bin on the same
  * arguments, workspace and stream, in one call: the forward's output plus the
  * binned workspace (and the parts of the three gradient buffers the binning
- * writes) that ms_deform_attn_backward_rest then consumes. Where the tile
- * path applies, the forward kernel itself stores the backward's records
+ * writes) that ms_deform_attn_backward_rest then consumes. Two forms with the
+ * same results: the forward kernel itself stores the backward's records
  * (bin_count and bin_scan run first, over the forward blocks' query chunks),
- * so the geometry is read once for both and nothing runs beside the forward;
- * elsewhere it makes exactly those two calls. Same results as the two calls.
+ * so the geometry is read once for both; or the binning's kernels, then the
+ * forward with the coarse levels in LDS. The call takes the faster one for
+ * its dims, or, where neither applies, makes exactly those two calls.
  * No reference counterpart: the reference forward
  * (/root/reference/csrc/ms_deformable_attn/ms_deform_attn_musa.mu:507-560)
  * prepares nothing for its backward. */
@@ -190,12 +191,13 @@ MUSPACE_API int ms_deform_attn_forward_bin(
     int64_t num_query, int64_t num_point, int64_t im2col_step, void *workspace,
     size_t workspace_bytes, void *stream);
 
-/* 1 if ms_deform_attn_forward_bin, given 16-byte-aligned tensors and a
- * 256-byte-aligned workspace of ms_deform_attn_backward_workspace_size bytes,
- * stores the backward's records from the forward kernel for these dims; 0 if
- * it runs ms_deform_attn_forward and the binning kernels instead (or the
- * shape takes the atomic backward). Results are the same either way. No
- * reference counterpart. */
+/* 1 if the forward kernel of ms_deform_attn_forward_bin, given 16-byte-aligned
+ * tensors and a 256-byte-aligned workspace of
+ * ms_deform_attn_backward_workspace_size bytes, can store the backward's
+ * records for these dims (large shapes take the other form all the same, where
+ * it is faster); 0 if the call runs ms_deform_attn_forward and the binning
+ * kernels (or the shape takes the atomic backward). Results are the same
+ * either way. No reference counterpart. */
 MUSPACE_API int ms_deform_attn_forward_bin_fused(int value_dtype, int64_t batch,
                                                  int64_t spatial_size, int64_t num_heads,
                                                  int64_t channels, int64_t num_levels,
@@ -323,7 +325,10 @@ MUSPACE_API int ms_deform_attn_backward_softmax_rest(
  * applies and each unit's L*P logits fit one step of the forward row kernel,
  * the softmax-fused forward kernel itself writes the probabilities and stores
  * the backward's records (weighted by the probabilities), as
- * ms_deform_attn_forward_bin does; elsewhere it makes exactly those two calls.
+ * ms_deform_attn_forward_bin does; where the binning's kernels and the forward
+ * with the coarse levels in LDS are faster (float32 geometry), these run, the
+ * forward on the stored probabilities; elsewhere it makes exactly those two
+ * calls.
  * Same contract as the two calls. No reference counterpart (the reference's
  * callers apply the softmax in torch before its forward). */
 MUSPACE_API int ms_deform_attn_forward_softmax_bin(
@@ -336,8 +341,9 @@ MUSPACE_API int ms_deform_attn_forward_softmax_bin(
     size_t workspace_bytes, void *stream);
 
 /* 1 if ms_deform_attn_forward_softmax_bin (aligned tensors, a workspace as
- * above) fuses the probabilities and the record stores into the forward kernel
- * for these dims; 0 if it makes the two calls. No reference counterpart. */
+ * above) can fuse the probabilities and the record stores into the forward
+ * kernel for these dims (large shapes take the other form where it is faster);
+ * 0 if it makes the two calls. No reference counterpart. */
 MUSPACE_API int ms_deform_attn_forward_softmax_bin_fused(int value_dtype, int64_t batch,
                                                          int64_t spatial_size,
                                                          int64_t num_heads, int64_t channels,

@@ -227,16 +227,17 @@ __device__ __forceinline__ void zero_boundary_cells(float *grad_value, size_t sl
   }
 }
 
-// Block-wide exclusive scan of per-thread run totals (kBinBlock threads);
+// Block-wide exclusive scan of per-thread run totals (kThreads threads);
 // returns this thread's offset, writes the grand total to *total. Only LDS
 // is exchanged, so the barriers leave global memory operations in flight.
+template <int kThreads = kBinBlock>
 __device__ __forceinline__ uint32_t block_exclusive(uint32_t run, uint32_t *part, uint32_t *total) {
   const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
   const uint32_t incl = wave_inclusive_sum(run);
   if (lane == kWave - 1) part[wid] = incl;
   lds_barrier();
   uint32_t before = 0, all = 0;
-  for (int w = 0; w < kBinBlock / kWave; ++w) {
+  for (int w = 0; w < kThreads / kWave; ++w) {
     const uint32_t v = part[w];
     before += w < wid ? v : 0u;
     all += v;
@@ -570,22 +571,28 @@ __global__ void __launch_bounds__(kBinBlock)
 
 // Samples per sub-chunk of bin_scatter (a power of two; the chunk's queries
 // are processed kScatterSlots >> lp_log2 at a time).
-constexpr int kScatterSlots = 2048;
-constexpr int kScatterPerThread = kScatterSlots / kBinBlock;
+constexpr int kScatterSlots = 4096;
+constexpr int kScatterPerThread = 8;
+constexpr int kScatterBlock = kScatterSlots / kScatterPerThread;
 
 __host__ __device__ constexpr size_t scatter_lds_bytes(int tile_bound) {
-  return static_cast<size_t>(kScatterSlots) * 16 +       // records in arrival order
-         static_cast<size_t>(kScatterSlots) * 4 +        // tile-sorted slot list
-         static_cast<size_t>(2 * (tile_bound + 1)) * 4;  // write cursors, local offsets
+  return static_cast<size_t>(kScatterSlots) * 8 +               // half records in tile order
+         static_cast<size_t>(kScatterSlots) * 2 +               // tile of each
+         static_cast<size_t>(tile_bound + 1) * 4 +              // write cursors
+         (static_cast<size_t>(tile_bound + 2) / 2 * 4);         // 16-bit counts, then offsets
 }
 
 // Writes each sample's 16-byte record into its tile's range and its record
-// index into the sample -> record map. A sub-chunk's records are first
-// ranked per tile and staged in LDS in arrival order, then written out in
-// tile order, so consecutive threads store consecutive records of one
-// tile's run (whole lines instead of one scattered 16-byte piece per lane).
+// index into the sample -> record map. A sub-chunk's records are ranked per
+// tile, then exchanged through LDS into tile order, half a record at a time,
+// and written out by consecutive threads, so that these store consecutive
+// records of one tile's run (whole lines instead of one scattered 16-byte
+// piece per lane). The kernel waits for its loads, atomics and barriers, so
+// what a workgroup holds in LDS sets its rate: half records and 16-bit
+// counters leave room for four workgroups a CU at the SCA shape where whole
+// records, a slot list and 32-bit counters left two.
 template <typename GT, int C, int T>
-__global__ void __launch_bounds__(kBinBlock)
+__global__ void __launch_bounds__(kScatterBlock, 4)
     msda_bin_scatter(const int64_t *__restrict__ shapes, const int64_t *__restrict__ starts,
                      const GT *__restrict__ loc, const GT *__restrict__ attn, Shape s, BinPlan p,
                      const uint32_t *__restrict__ counts,
@@ -596,12 +603,13 @@ __global__ void __launch_bounds__(kBinBlock)
                      float *__restrict__ grad_value) {
   __shared__ Level lv[kMaxLevels];
   __shared__ int ntc[kMaxLevels], base[kMaxLevels + 1];
-  __shared__ uint32_t part[kBinBlock / kWave];
+  __shared__ uint32_t part[kScatterBlock / kWave];
   extern __shared__ __align__(16) unsigned char dyn[];
-  uint4 *stage = reinterpret_cast<uint4 *>(dyn);                       // [kScatterSlots]
-  uint32_t *sorted = reinterpret_cast<uint32_t *>(stage + kScatterSlots);  // [kScatterSlots]
-  uint32_t *cursor = sorted + kScatterSlots;                         // [tile_bound + 1]
-  uint32_t *loff = cursor + (p.tile_bound + 1);                      // [tile_bound + 1]
+  uint2 *half = reinterpret_cast<uint2 *>(dyn);                          // [kScatterSlots]
+  uint32_t *cursor = reinterpret_cast<uint32_t *>(half + kScatterSlots);  // [tile_bound + 1]
+  uint32_t *counter = cursor + (p.tile_bound + 1);  // 16-bit, two a word: [tile_bound + 1]
+  uint16_t *loff = reinterpret_cast<uint16_t *>(counter);
+  uint16_t *tile_of = reinterpret_cast<uint16_t *>(counter + (p.tile_bound + 2) / 2);
   stage_levels(lv, shapes, starts, s);
   stage_tiles<T>(lv, s.levels, ntc, base);
   const int nt = base[s.levels];
@@ -617,21 +625,21 @@ __global__ void __launch_bounds__(kBinBlock)
   const int lpp = 1 << p.lp_log2;
   const int sub_q = kScatterSlots >> p.lp_log2;  // >= 1 (lpp <= kScatterSlots, checked on the host)
   // each thread owns a contiguous run of tiles in the scans below
-  const int per = (nt + kBinBlock - 1) / kBinBlock;
+  const int per = (nt + kScatterBlock - 1) / kScatterBlock;
   const int t0 = min(nt, static_cast<int>(threadIdx.x) * per), t1 = min(nt, t0 + per);
 
   for (int qs = 0; qs < nq; qs += sub_q) {
     const int nsq = min(sub_q, nq - qs);
-    for (int i = threadIdx.x; i < nt; i += blockDim.x) loff[i] = 0;
+    for (int i = threadIdx.x; i < (nt + 2) / 2; i += blockDim.x) counter[i] = 0;
     lds_barrier();
     // 1. loads first (every one unconditional, clamped index), then the tap,
-    // the rank inside its tile (LDS counter) and the record in arrival order
+    // the rank inside its tile (LDS counter) and the record
     float lx[kScatterPerThread], ly[kScatterPerThread], aw[kScatterPerThread];
-    uint32_t key[kScatterPerThread];  // tile << 12 | slot, or kNoRecord
-    uint32_t rk[kScatterPerThread];   // rank inside the tile
+    uint32_t id[kScatterPerThread];
+    uint32_t key[kScatterPerThread];  // tile << 16 | rank inside the tile, or kNoRecord
 #pragma unroll
     for (int u = 0; u < kScatterPerThread; ++u) {
-      const int j = threadIdx.x + u * kBinBlock;  // slot: query j >> lp_log2, sample j & (lpp - 1)
+      const int j = threadIdx.x + u * kScatterBlock;  // slot: query j >> lp_log2, sample j & (lpp - 1)
       const int q = q0 + qs + (j >> p.lp_log2), smp = j & (lpp - 1);
       const bool live = (j >> p.lp_log2) < nsq && smp < s.lp;
       const size_t o =
@@ -642,28 +650,26 @@ __global__ void __launch_bounds__(kBinBlock)
     }
 #pragma unroll
     for (int u = 0; u < kScatterPerThread; ++u) {
-      const int j = threadIdx.x + u * kBinBlock;
+      const int j = threadIdx.x + u * kScatterBlock;
       const int q = q0 + qs + (j >> p.lp_log2), smp = j & (lpp - 1);
       const bool live = (j >> p.lp_log2) < nsq && smp < s.lp;
       const int l = level_of_sample(live ? smp : 0, s);
       const Tap t = make_tap(lx[u], ly[u], lv[l], live);
       key[u] = kNoRecord;
-      rk[u] = 0;
       uint32_t at = kNoRecord;
       if (t.in) {
         const int tile = primary_tile<T>(t, ntc[l], base[l]);
-        const uint32_t rank = atomicAdd(&loff[tile], 1u);
-        key[u] = (static_cast<uint32_t>(tile) << 12) | static_cast<uint32_t>(j);
+        const int shift = (tile & 1) << 4;
+        const uint32_t rank = (atomicAdd(&counter[tile >> 1], 1u << shift) >> shift) & 0xffffu;
+        key[u] = (static_cast<uint32_t>(tile) << 16) | rank;
         at = cursor[tile] + rank;
         // top-left corner in the frame of its primary tile: [-1, T-1]^2 -> [0, T]^2
         const int ty = t.y0 < 0 ? 0 : t.y0, tx = t.x0 < 0 ? 0 : t.x0;
         const int pos = (t.y0 - (ty / T) * T + 1) * (T + 1) + (t.x0 - (tx / T) * T + 1);
-        stage[j] = make_uint4((static_cast<uint32_t>(pos) << kPosShift) |
-                                  (static_cast<uint32_t>(q) << p.lp_log2) |
-                                  static_cast<uint32_t>(smp),
-                              __float_as_uint(t.wx1), __float_as_uint(t.wy1),
-                              __float_as_uint(aw[u]));
-        rk[u] = rank;
+        id[u] = (static_cast<uint32_t>(pos) << kPosShift) |
+                (static_cast<uint32_t>(q) << p.lp_log2) | static_cast<uint32_t>(smp);
+        lx[u] = t.wx1;
+        ly[u] = t.wy1;
       }
       if (live) {
         const size_t o = (static_cast<size_t>(b * s.queries + q) * s.heads + m) * s.lp + smp;
@@ -681,31 +687,53 @@ __global__ void __launch_bounds__(kBinBlock)
     uint32_t run = 0;
     for (int t = t0; t < t1; ++t) run += loff[t];
     uint32_t total;
-    uint32_t off = block_exclusive(run, part, &total);
+    uint32_t off = block_exclusive<kScatterBlock>(run, part, &total);
     for (int t = t0; t < t1; ++t) {
       const uint32_t n = loff[t];
-      loff[t] = off;
+      loff[t] = static_cast<uint16_t>(off);
       off += n;
     }
-    if (threadIdx.x == 0) loff[nt] = total;
+    if (threadIdx.x == 0) loff[nt] = static_cast<uint16_t>(total);
     lds_barrier();
-    // 3. tile-sorted list of slots
+    // 3. first halves into tile order
 #pragma unroll
     for (int u = 0; u < kScatterPerThread; ++u) {
-      if (key[u] != kNoRecord) sorted[loff[key[u] >> 12] + rk[u]] = key[u];
+      if (key[u] != kNoRecord) {
+        const uint32_t tile = key[u] >> 16;
+        key[u] = loff[tile] + (key[u] & 0xffffu);  // from here on the record's place
+        tile_of[key[u]] = static_cast<uint16_t>(tile);
+        half[key[u]] = make_uint2(id[u], __float_as_uint(lx[u]));
+      }
     }
     lds_barrier();
-    // 4. records out in tile order: consecutive i of one tile are consecutive
-    // records of its global range
-    for (int i = threadIdx.x; i < static_cast<int>(total); i += kBinBlock) {
-      const uint32_t e = sorted[i];
-      const uint32_t tile = e >> 12, j = e & 0xfffu;
-      rec[cursor[tile] + (static_cast<uint32_t>(i) - loff[tile])] = stage[j];
+    // 4. the records of places threadIdx.x + u * kScatterBlock: where each goes, and
+    // its halves
+    uint2 lo[kScatterPerThread];
+    uint32_t dst[kScatterPerThread];
+#pragma unroll
+    for (int u = 0; u < kScatterPerThread; ++u) {
+      const uint32_t i = threadIdx.x + u * kScatterBlock;
+      const uint32_t tile = i < total ? tile_of[i] : 0u;
+      lo[u] = half[i];
+      dst[u] = cursor[tile] + (i - loff[tile]);
     }
     lds_barrier();
-    // 5. cursors past this sub-chunk's records
+#pragma unroll
+    for (int u = 0; u < kScatterPerThread; ++u) {
+      if (key[u] != kNoRecord) {
+        half[key[u]] = make_uint2(__float_as_uint(ly[u]), __float_as_uint(aw[u]));
+      }
+    }
+    // ... and the cursors past this sub-chunk's records
     for (int t = threadIdx.x; t < nt; t += blockDim.x) cursor[t] += loff[t + 1] - loff[t];
     lds_barrier();
+#pragma unroll
+    for (int u = 0; u < kScatterPerThread; ++u) {
+      const uint32_t i = threadIdx.x + u * kScatterBlock;
+      const uint2 hi = half[i];
+      if (i < total) store_nt(rec + dst[u], make_uint4(lo[u].x, lo[u].y, hi.x, hi.y));
+    }
+    lds_barrier();  // counters and halves are free
   }
 
   // non-boundary cells of the slab's empty and split tiles listed by

@@ -21,6 +21,7 @@
 #include "capi_errors.hpp"
 #include "msda_backward_tiles.hpp"
 #include "msda_forward_bin.hpp"
+#include "msda_forward_slab.hpp"
 #include "msda_kernels.hpp"
 
 namespace {
@@ -98,6 +99,16 @@ int validate(const char *fn, const Args &a, int value_dtype, int geometry_dtype,
   s.units = static_cast<int>(a.batch * a.queries * a.heads);
   s.inv_points = a.points > 0 ? 1.0f / static_cast<float>(a.points) : 0.0f;
   return ok();
+}
+
+// Dynamic LDS past the default limit of 64 KB has to be asked for.
+template <typename Kernel>
+void allow_lds(Kernel k, size_t bytes) {
+  if (bytes > 64 * 1024) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k),
+                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                              static_cast<int>(bytes));
+  }
 }
 
 int pow2_ceil(int v) {
@@ -219,6 +230,78 @@ void forward_rows_ns(const msda::Shape &s, Go &&go) {
   }
 }
 
+// Launch plan of the slab forward (msda_forward_slab.hpp).
+struct SlabLaunch {
+  bool ok = false;
+  bool narrow = false;  // 4 wavefronts a workgroup, two workgroups a CU
+  bool wide = false;    // several samples per geometry load
+  msda::SlabPlan plan{};
+};
+
+int slab_chunks(const SlabLaunch &L, int queries) {
+  return (queries + L.plan.chunk_q - 1) / L.plan.chunk_q;
+}
+
+// Whether a forward over `slabs` slabs of `queries` queries (for cameras: the
+// longest) takes the slab kernel, and its chunks.
+//
+// Workgroups of eight wavefronts, one a CU, in whole rounds over the 256 CUs. An
+// XCD's 32 CUs work on neighbouring chunks, so 32 chunks a slab keep it on one
+// slab, whose lines its L2 holds; where two heads share a 128-byte line (rows of
+// 64 bytes), 16 keep it on two heads' slabs. At the SCA shape fp32 took 579, 412,
+// 325 and 385 us at 8, 16, 32 and 48 chunks, bf16 227, 275 and 309 at 16, 32 and
+// 48; 3 x 8 slabs of 10007 fp16 queries 60 us at 16 (a round and a half), 54 at
+// 20. A workgroup copies the coarse levels (up to 119 KB) first, which 4096
+// samples and more pay for (the smallest measured have 5700).
+//
+// With one level there is nothing to copy, and workgroups of four wavefronts and
+// about 2048 of them are best (200 x 200 cells, 2 x 40000 queries, fp32: 83 us;
+// eight wavefronts: 112, 94 and 88 us at 32, 48 and 64 chunks).
+SlabLaunch plan_slab(const msda::Shape &s, int64_t slabs, int queries, size_t elem) {
+  SlabLaunch L;
+  if (s.lp < 4 || slabs <= 0 || queries <= 0) return L;
+  L.narrow = s.levels == 1;
+  const int64_t cus = 256;
+  const int64_t per_slab = s.channels * elem >= 128 ? 32 : 16;
+  int64_t rounds = L.narrow ? 8 : (slabs * per_slab + cus / 2) / cus;
+  if (rounds < 1) rounds = 1;
+  int64_t chunks = cus * rounds / slabs;
+  if (chunks < 1) chunks = 1;
+  L.plan.chunk_q = static_cast<int>((queries + chunks - 1) / chunks);
+  L.ok = static_cast<int64_t>(L.plan.chunk_q) * s.lp >= (L.narrow ? 1024 : 4096);
+  // wide loads where every block of NS * EP = 16 samples is whole and a pair of
+  // samples seldom straddles two levels (at 16 samples of 4 points: 109 against
+  // 99 us)
+  L.wide = s.lp >= 32 && s.lp % 16 == 0;
+  return L;
+}
+
+template <typename VT, typename GT, int C, typename Out>
+void launch_slab(const VT *v, uint32_t vbytes, const int64_t *shapes, const int64_t *starts,
+                 const GT *lc, const GT *aw, const Out &out, const msda::Shape &s,
+                 const SlabLaunch &L, int blocks, hipStream_t st) {
+  auto go = [&](auto wc, auto ec) {
+    constexpr int W = decltype(wc)::value, EP = decltype(ec)::value;
+    using Cfg = msda::SlabCfg<VT, C, W>;
+    auto k = msda::msda_forward_slab<VT, GT, C, W, EP, Out>;
+    allow_lds(k, Cfg::kLds);
+    k<<<blocks, Cfg::kBlock, Cfg::kLds, st>>>(v, vbytes, shapes, starts, lc, aw, out, s, L.plan);
+  };
+  using One = std::integral_constant<int, 1>;
+  if constexpr (std::is_same<Out, msda::DenseRows<VT>>::value) {
+    if (L.narrow) {
+      go(std::integral_constant<int, 4>(), One());
+      return;
+    }
+  }
+  if (L.wide) {
+    go(std::integral_constant<int, 8>(),
+       std::integral_constant<int, 16 / msda::SlabCfg<VT, C, 8>::NS>());
+  } else {
+    go(std::integral_constant<int, 8>(), One());
+  }
+}
+
 template <typename VT, typename GT, int C>
 void launch_forward_rows(const void *value, const int64_t *shapes, const int64_t *starts,
                          const void *loc, const void *attn, void *out, const msda::Shape &s,
@@ -228,6 +311,14 @@ void launch_forward_rows(const void *value, const int64_t *shapes, const int64_t
   const GT *aw = static_cast<const GT *>(attn);
   VT *o = static_cast<VT *>(out);
   const uint32_t vbytes = static_cast<uint32_t>(value_bytes(s, sizeof(VT)));
+  if constexpr (C == 32 || C == 64) {
+    const SlabLaunch L = plan_slab(s, static_cast<int64_t>(s.batch) * s.heads, s.queries, sizeof(VT));
+    if (L.ok) {
+      launch_slab<VT, GT, C>(v, vbytes, shapes, starts, lc, aw, msda::DenseRows<VT>{o}, s, L,
+                             slab_chunks(L, s.queries) * s.batch * s.heads, st);
+      return;
+    }
+  }
   forward_rows_ns<VT, C>(s, [&](auto ns, const Launch &L) {
     msda::msda_forward_rows<VT, GT, C, decltype(ns)::value>
         <<<L.blocks, msda::kBlock, 0, st>>>(v, vbytes, shapes, starts, lc, aw, o, s, L.plan);
@@ -417,6 +508,27 @@ void launch_scatter_div(const void *value, const int64_t *shapes, const int64_t 
   auto go = [&](auto cc) {
     constexpr int C = decltype(cc)::value;
     constexpr int KQ = C / msda::RowTraits<VT>::kCpl;
+    if constexpr (C == 32 || C == 64) {
+      int longest = 0;
+      for (int j = 0; j < out.ncam; ++j) {
+        const int len = out.off[j + 1] - out.off[j];
+        longest = len > longest ? len : longest;
+      }
+      const int64_t slabs = static_cast<int64_t>(s.batch) * s.heads;
+      const SlabLaunch L = plan_slab(s, slabs * out.ncam, longest, sizeof(VT));
+      if (L.ok) {
+        msda::CameraSlots<VT, GT, kAtomic> seg = out;
+        int64_t blocks = 0;
+        for (int j = 0; j < seg.ncam; ++j) {
+          seg.blk[j] = static_cast<int>(blocks);
+          blocks += slabs * slab_chunks(L, seg.off[j + 1] - seg.off[j]);
+        }
+        seg.blk[seg.ncam] = static_cast<int>(blocks);
+        launch_slab<VT, GT, C>(v, vbytes, shapes, starts, lc, aw, seg, s, L,
+                               static_cast<int>(blocks), st);
+        return;
+      }
+    }
     forward_rows_ns<VT, C>(s, [&](auto ns, const Launch &L) {
       // one segment of whole blocks per camera (the plan depends on L*P only)
       msda::CameraSlots<VT, GT, kAtomic> seg = out;
@@ -697,10 +809,10 @@ bool plan_tile_workspace(const msda::Shape &s, int value_dtype, TileWorkspace &w
   const int64_t bound = static_cast<int64_t>(s.spatial) / T + s.levels + 1;
   if (bound > msda::kMaxTilesPerSlab) return false;
   p.tile_bound = static_cast<int>(bound);
-  // bin_scatter stages a sub-chunk of records and two tile arrays in LDS
-  if (msda::scatter_lds_bytes(p.tile_bound) + 4096 > msda::kTileLdsLimit) return false;
+  // the binning kernels' LDS tables of a word per tile (bin_count's the largest)
+  if (bound > 14847) return false;
   p.lp_log2 = log2_int(s.lp > 0 ? s.lp : 1);
-  if ((1 << p.lp_log2) > msda::kScatterSlots) return false;
+  if ((1 << p.lp_log2) > 2048) return false;
   // record ids pack (q << lp_log2) | sample below bit kPosShift and the tap's
   // position in the tile frame above it
   if ((static_cast<int64_t>(s.queries) << p.lp_log2) > (int64_t{1} << msda::kPosShift)) return false;
@@ -797,13 +909,10 @@ void launch_backward_tiles(const void *value, const int64_t *shapes, const int64
   auto scatter = msda::msda_bin_scatter<GT, C, T>;
   auto tile = msda::msda_tile_backward<VT, C>;
   constexpr size_t tile_bytes = msda::tile_lds_bytes<VT, C>();
-  (void)hipFuncSetAttribute(reinterpret_cast<const void *>(count),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, hist_bytes);
+  allow_lds(count, hist_bytes);
   const size_t scatter_bytes = msda::scatter_lds_bytes(p.tile_bound);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void *>(scatter),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, scatter_bytes);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void *>(tile),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, tile_bytes);
+  allow_lds(scatter, scatter_bytes);
+  allow_lds(tile, tile_bytes);
 
   if (phase != Phase::kRest) {
     count<<<bm * count_groups(p), msda::kBinBlock, hist_bytes, st>>>(shapes, starts, lc, s, p,
@@ -811,7 +920,7 @@ void launch_backward_tiles(const void *value, const int64_t *shapes, const int64
     launch_bin_cursors<T>(shapes, starts, s, p, bm, counts, tile_start, st);
     msda::msda_bin_scan<C, T><<<bm, msda::kBinBlock, 0, st>>>(
         shapes, starts, s, p, tile_start, item_total, items, zero_tiles, gv);
-    scatter<<<bm * p.chunks, msda::kBinBlock, scatter_bytes, st>>>(
+    scatter<<<bm * p.chunks, msda::kScatterBlock, scatter_bytes, st>>>(
         shapes, starts, lc, aw, s, p, counts, tile_start, zero_tiles, records, rec_of_sample, gl,
         ga, gv);
   }
@@ -847,6 +956,20 @@ bool fwd_bin_fuses(const msda::Shape &s, int value_dtype, const TileWorkspace &w
   if (softmax && unit_steps != 1) return false;
   return slots <= msda::kFwdBinSlots &&
          msda::fwd_bin_lds_bytes(slots, w.plan.tile_bound) <= msda::kFwdBinDynLds;
+}
+
+// Whether a forward with binning runs the slab forward and the binning kernels
+// although the row kernel could store the records itself. Both forms, forward
+// call and tile kernel together: encoder 2 x 22223 queries, 16 samples fp32 405 ->
+// 383 us; one 200 x 200 level fp32 300 -> 293 us; SCA 12 x 15000 queries, 32
+// samples bf16 2804 -> 2675 us. At 6 x 10000 queries, 32 samples fp32 they are
+// within 1%, and the row kernel stays there: with uniform locations a workgroup's
+// records of a fine tile are short runs, which the binning kernels' scatter pays
+// more for (159 us), and in fp32 only the smallest level fits the LDS.
+bool bins_apart(const msda::Shape &s, size_t elem) {
+  if (s.channels != 32 && s.channels != 64) return false;
+  if (elem == 4 && s.lp >= 32) return false;
+  return plan_slab(s, static_cast<int64_t>(s.batch) * s.heads, s.queries, elem).ok;
 }
 
 // The forward with the backward's binning fused in (msda_forward_bin.hpp):
@@ -892,8 +1015,7 @@ bool launch_forward_bin_tiles(const void *value, const int64_t *shapes, const in
   const GT *aw = static_cast<const GT *>(attn);
   const size_t hist_bytes = count_hist_bytes(p);
   auto count = msda::msda_bin_count<GT, C, T>;
-  (void)hipFuncSetAttribute(reinterpret_cast<const void *>(count),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, hist_bytes);
+  allow_lds(count, hist_bytes);
   count<<<bm * count_groups(p), msda::kBinBlock, hist_bytes, st>>>(shapes, starts, lc, s, p,
                                                                    counts, item_total, gv);
   launch_bin_cursors<T>(shapes, starts, s, p, bm, counts, tile_start, st);
@@ -906,8 +1028,7 @@ bool launch_forward_bin_tiles(const void *value, const int64_t *shapes, const in
   forward_rows_ns<VT, C>(s, [&](auto ns, const Launch &L) {
     auto k = probs ? msda::msda_forward_softmax_bin_rows<VT, GT, C, decltype(ns)::value, T>
                    : msda::msda_forward_bin_rows<VT, GT, C, decltype(ns)::value, T>;
-    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    allow_lds(k, lds);
     k<<<bm * p.chunks, msda::kBlock, lds, st>>>(static_cast<const VT *>(value), vbytes, shapes,
                                                  starts, lc, aw, static_cast<VT *>(out), s,
                                                  L.plan, args);
@@ -927,6 +1048,9 @@ bool launch_forward_bin(const void *value, const int64_t *shapes, const int64_t 
                     workspace_bytes >= w.bytes && rows_aligned({value, out, gv}, gl) &&
                     aligned(workspace, 256);
   if (!fits) return false;
+  // apart, a softmax forward reads the stored probabilities: not where these are
+  // narrower than the float32 ones of the fused forward
+  if (bins_apart(s, sizeof(VT)) && !(probs && sizeof(GT) < 4)) return false;
   switch (s.channels) {
     case 16:
       return launch_forward_bin_tiles<VT, GT, 16>(value, shapes, starts, loc, attn, out, gv, gl,
@@ -1418,19 +1542,20 @@ int ms_deform_attn_forward_bin(const void *value, int value_dtype, const int64_t
     });
     if (fused) return check_launch(fn);
   }
-  // the two calls this one stands for
-  if (int rc = ms_deform_attn_forward(value, value_dtype, spatial_shapes, level_start_index,
-                                      sampling_locations, attention_weights, geometry_dtype,
-                                      output, batch, spatial_size, num_heads, channels,
-                                      num_levels, num_query, num_point, im2col_step, stream)) {
+  // the two calls this one stands for, the binning first: the backward's next
+  // kernel then finds the value where the forward left it
+  if (int rc = ms_deform_attn_backward_bin(value, value_dtype, spatial_shapes, level_start_index,
+                                           sampling_locations, attention_weights, geometry_dtype,
+                                           nullptr, grad_value, grad_sampling_locations,
+                                           grad_attention_weights, batch, spatial_size, num_heads,
+                                           channels, num_levels, num_query, num_point,
+                                           im2col_step, workspace, workspace_bytes, stream)) {
     return rc;
   }
-  return ms_deform_attn_backward_bin(value, value_dtype, spatial_shapes, level_start_index,
-                                     sampling_locations, attention_weights, geometry_dtype,
-                                     nullptr, grad_value, grad_sampling_locations,
-                                     grad_attention_weights, batch, spatial_size, num_heads,
-                                     channels, num_levels, num_query, num_point, im2col_step,
-                                     workspace, workspace_bytes, stream);
+  return ms_deform_attn_forward(value, value_dtype, spatial_shapes, level_start_index,
+                                sampling_locations, attention_weights, geometry_dtype, output,
+                                batch, spatial_size, num_heads, channels, num_levels, num_query,
+                                num_point, im2col_step, stream);
 }
 
 int ms_deform_attn_backward(const void *value, int value_dtype, const int64_t *spatial_shapes,
@@ -1634,6 +1759,23 @@ int ms_deform_attn_forward_softmax_bin(
     });
     if (fused) return check_launch(fn);
   }
+  auto bin = [&] {
+    return ms_deform_attn_backward_softmax_bin(
+        value, value_dtype, spatial_shapes, level_start_index, sampling_locations,
+        attention_logits, geometry_dtype, nullptr, grad_value, grad_sampling_locations,
+        grad_attention_logits, batch, spatial_size, num_heads, channels, num_levels, num_query,
+        num_point, im2col_step, workspace, workspace_bytes, stream);
+  };
+  if (needs_data(s) && s.lp > 0 && geometry_dtype == MUSPACE_DTYPE_F32 &&
+      bins_apart(s, value_dtype == MUSPACE_DTYPE_F32 ? 4 : 2)) {
+    // the binning's probabilities, at the head of the workspace, are the slab
+    // forward's weights
+    if (int rc = bin()) return rc;
+    return ms_deform_attn_forward(value, value_dtype, spatial_shapes, level_start_index,
+                                  sampling_locations, workspace, geometry_dtype, output, batch,
+                                  spatial_size, num_heads, channels, num_levels, num_query,
+                                  num_point, im2col_step, stream);
+  }
   // the two calls this one stands for
   if (int rc = ms_deform_attn_forward_softmax(value, value_dtype, spatial_shapes,
                                               level_start_index, sampling_locations,
@@ -1642,11 +1784,7 @@ int ms_deform_attn_forward_softmax_bin(
                                               num_query, num_point, im2col_step, stream)) {
     return rc;
   }
-  return ms_deform_attn_backward_softmax_bin(
-      value, value_dtype, spatial_shapes, level_start_index, sampling_locations,
-      attention_logits, geometry_dtype, nullptr, grad_value, grad_sampling_locations,
-      grad_attention_logits, batch, spatial_size, num_heads, channels, num_levels, num_query,
-      num_point, im2col_step, workspace, workspace_bytes, stream);
+  return bin();
 }
 
 int ms_deform_attn_forward_softmax_bin_fused(int value_dtype, int64_t batch,

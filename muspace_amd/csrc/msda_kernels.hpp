@@ -97,6 +97,8 @@ struct DenseRows {
     row = (b * s.queries + q) * s.heads + m;
     slab = static_cast<size_t>(b) * s.spatial;
   }
+  // one segment: all blocks, all queries (CameraSlots cuts them by camera)
+  __device__ __forceinline__ const DenseRows &segment(int &, Shape &) const { return *this; }
   // what the epilogue of a unit loads ahead of time (nothing here)
   static constexpr bool kLoadsAhead = false;
   struct Ticket {};

@@ -134,9 +134,10 @@ def _native_geometry_dtype(value: torch.Tensor, *geometry: torch.Tensor) -> torc
 # Early binning: the tile-owned backward's binning reads only the geometry, so
 # the forward does it. ms_deform_attn_forward_bin runs the forward and the
 # binning as one call, in which the forward kernel itself stores the
-# backward's records (the geometry is read once for both; a binning on a second
-# stream beside the forward kernel could not overlap it, the forward's
-# registers leaving no room on its SIMDs). The backward's buffers (its scratch
+# backward's records, or the binning's kernels run right before it, whichever is
+# faster for the shape (a binning on a second stream beside the forward kernel
+# could not overlap it, the forward's registers leaving no room on its SIMDs).
+# The backward's buffers (its scratch
 # and the three float32 gradients) then live from the forward to the
 # backward; MUSPACE_EARLY_BINNING=0 turns this off, and a per-device byte
 # budget bounds what all forwards awaiting their backward may hold

@@ -518,19 +518,21 @@ class NativeLibrary:
         return self._workspace_bytes(value, sampling_locations, softmax=True)
 
     def forward_bin_fuses(self, value, sampling_locations) -> bool:
-        """Whether :meth:`ms_deform_attn_forward_bin` stores the backward's
-        records from the forward kernel for these shapes (else it runs the
-        plain forward and the binning kernels; same results)."""
+        """Whether the forward kernel of :meth:`ms_deform_attn_forward_bin` can
+        store the backward's records for these shapes (it does where that is
+        the faster form; else the call runs the plain forward and the binning
+        kernels; same results)."""
         batch, spatial, heads, channels = value.shape
         _, queries, _, levels, points, _ = sampling_locations.shape
         return bool(self._raw["ms_deform_attn_forward_bin_fused"](
             _dtype_code(value.dtype), batch, spatial, heads, channels, levels, queries, points))
 
     def forward_softmax_bin_fuses(self, value, sampling_locations) -> bool:
-        """Whether :meth:`ms_deform_attn_forward_softmax_bin` writes the
-        probabilities and stores the backward's records from the softmax-fused
-        forward kernel for these shapes (else it runs the softmax forward and
-        the softmax binning; same results)."""
+        """Whether the softmax-fused forward kernel of
+        :meth:`ms_deform_attn_forward_softmax_bin` can write the probabilities
+        and store the backward's records for these shapes (it does where that
+        is the faster form; else the call runs a forward and the softmax
+        binning; same results)."""
         batch, spatial, heads, channels = value.shape
         _, queries, _, levels, points, _ = sampling_locations.shape
         return bool(self._raw["ms_deform_attn_forward_softmax_bin_fused"](
