@@ -171,14 +171,16 @@ __global__ void __launch_bounds__(W * kWave, kRowWavesPerSimd)
   // geometry of this lane's EP samples of a block
   struct Geometry {
     float xy[2 * EP], a[EP];
-    int smp;  // the first sample; -1: none
+    int smp;  // the first sample
+    bool ok;  // in the chunk and below L*P
   };
   int gb = 0, gq = q0 + wave * NG + tg;  // the next block to load, and its query
   auto load_geometry = [&]() __attribute__((always_inline)) {
     Geometry g;
     const int smp = gb * NS * EP + tj * EP;
     const bool ok = gq < q1 && lane < NG * NS && smp < s.lp;
-    g.smp = ok ? smp : -1;
+    g.smp = smp;
+    g.ok = ok;
     const size_t o =
         static_cast<size_t>(row0 + (ok ? gq : 0) * s.heads) * s.lp + (ok ? smp : 0);
     if constexpr (sizeof(GT) == 4) {
@@ -204,8 +206,9 @@ __global__ void __launch_bounds__(W * kWave, kRowWavesPerSimd)
   };
   // this lane's tap of its e-th sample into table `par`
   auto tap = [&](const Geometry &g, int e, int par) __attribute__((always_inline)) {
-    const bool ok = g.smp >= 0;
-    const int smp = ok ? g.smp + e : 0;
+    const bool ok = g.ok;
+    // a unit past the chunk keeps its sample's place: consume picks LDS or L2 by it
+    const int smp = min(g.smp + e, s.lp - 1);
     const int l = level_of_sample(smp, s);
     const Level L = lv[l];
     const Tap t = make_tap(g.xy[2 * e], g.xy[2 * e + 1], L, ok);
@@ -231,8 +234,8 @@ __global__ void __launch_bounds__(W * kWave, kRowWavesPerSimd)
   };
   // Samples of stage h of pass (block bk of its unit, e): sample index of the
   // stage's j-th; uniform, so what a sample gathers from is a scalar branch.
-  // A sample past L*P is skipped; a unit past the chunk has zero weights and,
-  // with none of its offsets inside, reads zeros.
+  // A sample past L*P is skipped; a unit past the chunk has zero weights and
+  // reads zeros: the zero row of the LDS, or past the value buffer's end.
   auto sample_of = [&](int bk, int e, int h, int j) {
     return bk * NS * EP + (h * NH + j) * EP + e;
   };
