@@ -87,6 +87,8 @@ struct BinPlan {
   // (a chunk has fewer than 65536 samples), half the LDS, twice the blocks
   // per CU where the histograms limit them
   int hist16;
+  // 1: bin_scatter's record stores go through the L2; 0: past it
+  int merge_records;
 };
 
 // One work item: records [r0, r1) of one tile of the (b, m) slab. `tile`
@@ -587,10 +589,12 @@ __host__ __device__ constexpr size_t scatter_lds_bytes(int tile_bound) {
 // tile, then exchanged through LDS into tile order, half a record at a time,
 // and written out by consecutive threads, so that these store consecutive
 // records of one tile's run (whole lines instead of one scattered 16-byte
-// piece per lane). The kernel waits for its loads, atomics and barriers, so
-// what a workgroup holds in LDS sets its rate: half records and 16-bit
-// counters leave room for four workgroups a CU at the SCA shape where whole
-// records, a slot list and 32-bit counters left two.
+// piece per lane). The kernel waits for its loads, atomics and barriers; half
+// records and 16-bit counters let 16 wavefronts a CU (two workgroups, by their
+// 127 VGPRs) exchange 4096 records each in 42 KB. Encoder 2 x 22223 queries, 16
+// samples: 50 us; 12 x 15000 queries, 32 samples: 447-512 us. Three workgroups
+// at 80 VGPRs spill (118, 877 us); four slots a thread and 1024 threads, 72 and
+// 534 us.
 template <typename GT, int C, int T>
 __global__ void __launch_bounds__(kScatterBlock, 4)
     msda_bin_scatter(const int64_t *__restrict__ shapes, const int64_t *__restrict__ starts,
@@ -731,7 +735,12 @@ __global__ void __launch_bounds__(kScatterBlock, 4)
     for (int u = 0; u < kScatterPerThread; ++u) {
       const uint32_t i = threadIdx.x + u * kScatterBlock;
       const uint2 hi = half[i];
-      if (i < total) store_nt(rec + dst[u], make_uint4(lo[u].x, lo[u].y, hi.x, hi.y));
+      const uint4 r = make_uint4(lo[u].x, lo[u].y, hi.x, hi.y);
+      if (p.merge_records) {  // uniform
+        if (i < total) rec[dst[u]] = r;
+      } else {
+        if (i < total) store_nt(rec + dst[u], r);
+      }
     }
     lds_barrier();  // counters and halves are free
   }

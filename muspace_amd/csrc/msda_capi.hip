@@ -840,6 +840,16 @@ bool plan_tile_workspace(const msda::Shape &s, int value_dtype, TileWorkspace &w
   p.direct = p.rec_cap * 12 <= (8 << 20) ? 1 : 0;
   if (p.rec_cap >= (int64_t{1} << 31)) return false;
   const int64_t bm = static_cast<int64_t>(s.batch) * s.heads;
+  // bin_scatter ends a run of a tile's records in the middle of a line that the
+  // next run continues. While all records fit the 256 MB memory-side cache, that
+  // cache joins the pieces and the stores leave the L2 to the value rows the next
+  // kernels read; past it the pieces reach the HBM one by one, unless the L2 has
+  // joined them. Through the L2 against past it, bin_scatter (tile kernel): 737 MB
+  // of records (12 x 15000 queries, 32 samples, bf16) 439 against 515 us (1275,
+  // 1277); 246 MB (six cameras, 32 samples, fp32) 118, 134 (580, 559); 91 MB
+  // (2 x 22223, 16 samples) 52, 52 (192, 180); 41 MB (2 x 40000, 4 samples) 34, 33
+  // (135, 127).
+  p.merge_records = bm * p.rec_cap * 16 > (int64_t{256} << 20) ? 1 : 0;
   // records per work item (a tile with more is split into items whose cells
   // are all added atomically): about 4 items' worth per workgroup, 4 to 8
   // batches, in whole batches. Measured at the benchmark shapes: single-

@@ -164,3 +164,27 @@ def test_training_calls_that_bin_apart(vdt, gdt, softmax):
     for i in (2, 3):
         piece = torch.cat([p[i] for p in pieces], 1)
         torch.testing.assert_close(whole[i].float(), piece.float(), rtol=tol, atol=tol)
+
+
+def test_records_past_the_memory_side_cache():
+    """A batch whose binned records pass 256 MB (their stores then go through the L2)
+    gives what its entries give one by one. Outputs and location and weight
+    gradients are each one unit's or sample's own sum. A value gradient sums, in
+    another order, up to some 350 products (23000 queries x 4 samples x 4 corners over
+    1050 cells) whose magnitudes add up to about 9: 350 * 2^-24 * 9 = 1.9e-4 at worst."""
+    levels, queries, points, batch = ((60, 70), (30, 35)), 23000, 4, 12
+    value, shapes, starts, loc, logits = _inputs(11, levels, queries, points, batch=batch)
+    assert batch * queries * 8 * len(levels) * points * 16 > 256 << 20
+    attn = _weights(logits, F32)
+    grad = torch.randn(batch, queries, 256, generator=torch.Generator().manual_seed(12)).to(DEV)
+
+    def call(part):
+        leaves = [t[part].clone().requires_grad_() for t in (value, loc, attn)]
+        out = multi_scale_deformable_attn(leaves[0], shapes, starts, leaves[1], leaves[2])
+        return (out.detach(), *torch.autograd.grad(out, leaves, grad[part]))
+
+    whole = call(slice(None))
+    for entry in (0, 5, batch - 1):
+        one = call(slice(entry, entry + 1))
+        for i, atol in enumerate((1e-5, 2e-4, 1e-5, 1e-5)):
+            torch.testing.assert_close(whole[i][entry: entry + 1], one[i], rtol=1e-5, atol=atol)
