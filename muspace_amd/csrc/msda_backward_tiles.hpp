@@ -592,9 +592,10 @@ __host__ __device__ constexpr size_t scatter_lds_bytes(int tile_bound) {
 // piece per lane). The kernel waits for its loads, atomics and barriers; half
 // records and 16-bit counters let 16 wavefronts a CU (two workgroups, by their
 // 127 VGPRs) exchange 4096 records each in 42 KB. Encoder 2 x 22223 queries, 16
-// samples: 50 us; 12 x 15000 queries, 32 samples: 447-512 us. Three workgroups
-// at 80 VGPRs spill (118, 877 us); four slots a thread and 1024 threads, 72 and
-// 534 us.
+// samples: 50 us; 12 x 15000 queries, 32 samples: 439 us (512 with its stores
+// past the L2, BinPlan::merge_records). Before that change, three workgroups at
+// 80 VGPRs spilled (118 and 877 us), and four slots a thread in 1024 threads
+// took 72 and 534 us.
 template <typename GT, int C, int T>
 __global__ void __launch_bounds__(kScatterBlock, 4)
     msda_bin_scatter(const int64_t *__restrict__ shapes, const int64_t *__restrict__ starts,
