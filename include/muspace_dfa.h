@@ -83,10 +83,11 @@ MUSPACE_API int deformable_aggregation_backward_opt(
 /* The backward with grad_mc_ms_feat OVERWRITTEN (every element, zero where
  * nothing samples it) instead of added to. Given a workspace of at least
  * deformable_aggregation_backward_workspace_size bytes (0: the shape has no
- * such path; NULL is then fine), each feature row's contributions are listed
- * in it and summed once per row in float64, without atomics; else the
- * gradient is zeroed and taken as by backward_opt. Nothing is kept in the
- * workspace between calls. */
+ * such path; NULL is then fine), aligned to 256 bytes, each feature row's
+ * contributions are listed in it and summed once per row in float64, without
+ * atomics; else (no, a smaller or a misaligned workspace) the gradient is
+ * zeroed and taken as by backward_opt. Nothing is kept in the workspace between
+ * calls. */
 MUSPACE_API size_t deformable_aggregation_backward_workspace_size(
     int64_t batch, int64_t num_cams, int64_t num_feat, int64_t num_embeds, int64_t num_scale,
     int64_t num_anchors, int64_t num_pts, int64_t num_groups);

@@ -320,7 +320,9 @@ int backward_ws_impl(const char *fn, const float *feat, const int32_t *shape,
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   OwnerWorkspace w;
-  if (!sampled || !plan_owner(d, w) || !workspace || workspace_bytes < w.bytes) {
+  // the kernels read and write the workspace in pieces of up to 16 bytes
+  const bool aligned = reinterpret_cast<uintptr_t>(workspace) % 256 == 0;
+  if (!sampled || !plan_owner(d, w) || !workspace || workspace_bytes < w.bytes || !aligned) {
     if (n_feat > 0) {
       dfa::dfa_zero<<<generic_blocks(n_feat), dfa::kBlock, 0, st>>>(grad_feat, n_feat);
     }

@@ -143,6 +143,29 @@ def test_captured_backward_replays():
             torch.testing.assert_close(g, e, rtol=1e-6, atol=1e-6)
 
 
+@gpu
+@pytest.mark.parametrize("offset,short", [(0, 0), (8, 0), (128, 0), (1, 0), (0, 1)])
+def test_misaligned_or_short_workspace_is_left_alone(offset, short):
+    """A workspace off a 256-byte boundary, or a byte too small, takes the kernels
+    without one: right gradients, and not a byte of it written."""
+    case = [t.to(DEV) for t in _case(43, ((9, 13), (4, 6)), 256, 8, anchors=60)]
+    grad_out = torch.randn(2, 60, 256, generator=torch.Generator().manual_seed(44)).to(DEV)
+    lib = load_native_module()
+    dims = [2, 3, case[0].shape[1], 256, 2, 60, 3, 8]
+    size = lib.raw("deformable_aggregation_backward_workspace_size")(*dims)
+    workspace = torch.full((size + 256,), 0x5A, dtype=torch.uint8, device=DEV)
+    assert workspace.data_ptr() % 256 == 0
+    grads = [torch.full_like(case[i], float("nan")) for i in (0, 3, 4)]
+    code = lib.raw("deformable_aggregation_backward_ws")(
+        *[t.data_ptr() for t in (*case, grad_out, *grads)], *dims, workspace.data_ptr() + offset,
+        size - short, torch.cuda.current_stream().cuda_stream)
+    assert code == 0
+    assert bool((workspace == 0x5A).all()) == bool(offset or short)
+    expected = _backward(case, grad_out)
+    for g, e, atol in zip(grads, expected, (1e-5, 1e-3, 1e-4)):
+        torch.testing.assert_close(g.cpu(), e, rtol=1e-5, atol=atol)
+
+
 def test_workspace_size_and_validation(native_lib):
     size = native_lib.raw("deformable_aggregation_backward_workspace_size")
     dims = [2, 3, 500, 256, 2, 40, 4, 8]  # batch, cams, feat, embeds, scales, anchors, pts, groups
