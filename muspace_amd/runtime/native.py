@@ -895,8 +895,13 @@ class NativeLibrary:
         scratch = ()
         if with_workspace:
             nbytes = self._raw["deformable_aggregation_backward_workspace_size"](*dims)
-            workspace = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=mc_ms_feat.device)
-            scratch = (workspace.data_ptr(), nbytes)
+            try:
+                workspace = torch.empty(nbytes, dtype=torch.uint8, device=mc_ms_feat.device)
+                scratch = (workspace.data_ptr(), nbytes)
+            except torch.OutOfMemoryError:
+                # sized for every pair active, up to 8 GiB: the kernels with atomics
+                # need none of it
+                scratch = (None, 0)
         self._launch(
             name, mc_ms_feat.device,
             mc_ms_feat.data_ptr(), spatial_shape.data_ptr(), scale_start_index.data_ptr(),
@@ -931,7 +936,8 @@ class NativeLibrary:
                                         grad_mc_ms_feat, grad_sampling_location,
                                         grad_weights) -> None:
         """All three gradients overwritten (none needs zero-filling); the
-        scratch comes from torch's caching allocator."""
+        scratch comes from torch's caching allocator, and a call that cannot
+        have it takes the kernels without."""
         self._dfa_backward("deformable_aggregation_backward_ws", mc_ms_feat, spatial_shape,
                            scale_start_index, sampling_location, weights, grad_output,
                            grad_mc_ms_feat, grad_sampling_location, grad_weights,

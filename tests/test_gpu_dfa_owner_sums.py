@@ -166,6 +166,27 @@ def test_misaligned_or_short_workspace_is_left_alone(offset, short):
         torch.testing.assert_close(g.cpu(), e, rtol=1e-5, atol=atol)
 
 
+@gpu
+def test_scratch_that_cannot_be_had(monkeypatch):
+    """Out of memory for the scratch alone: the call takes the kernels without it."""
+    case = _case(45, ((9, 13), (4, 6)), 256, 8, anchors=60)
+    grad_out = torch.randn(2, 60, 256, generator=torch.Generator().manual_seed(46))
+    expected = _backward(case, grad_out)
+    asked, empty = [], torch.empty
+
+    def no_bytes(*args, **kwargs):
+        if kwargs.get("dtype") == torch.uint8:
+            asked.append(args)
+            raise torch.OutOfMemoryError("out of memory")
+        return empty(*args, **kwargs)
+
+    monkeypatch.setattr(torch, "empty", no_bytes)
+    actual = _backward(case, grad_out)
+    assert asked
+    for a, e, atol in zip(actual, expected, (1e-5, 1e-3, 1e-4)):
+        torch.testing.assert_close(a, e, rtol=1e-5, atol=atol)
+
+
 def test_workspace_size_and_validation(native_lib):
     size = native_lib.raw("deformable_aggregation_backward_workspace_size")
     dims = [2, 3, 500, 256, 2, 40, 4, 8]  # batch, cams, feat, embeds, scales, anchors, pts, groups
