@@ -92,6 +92,12 @@ MUSPACE_API size_t deformable_aggregation_backward_workspace_size(
     int64_t batch, int64_t num_cams, int64_t num_feat, int64_t num_embeds, int64_t num_scale,
     int64_t num_anchors, int64_t num_pts, int64_t num_groups);
 
+/* 1 where backward_ws is faster with its workspace than without (0 for one
+ * scale, and for large maps sampled at few points). */
+MUSPACE_API int deformable_aggregation_backward_prefers_workspace(
+    int64_t batch, int64_t num_cams, int64_t num_feat, int64_t num_embeds, int64_t num_scale,
+    int64_t num_anchors, int64_t num_pts, int64_t num_groups);
+
 MUSPACE_API int deformable_aggregation_backward_ws(
     const float *mc_ms_feat, const int32_t *spatial_shape, const int32_t *scale_start_index,
     const float *sampling_location, const float *weights, const float *grad_output,

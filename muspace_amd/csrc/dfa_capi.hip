@@ -302,6 +302,62 @@ bool plan_owner(const dfa::Dims &d, OwnerWorkspace &w) {
   return off <= (size_t{8} << 30);
 }
 
+// Feature rows of a workgroup in dfa_list_rows and dfa_sum_rows: powers of two,
+// sum_rows the smaller, so that a workgroup of the sums stays inside a range of
+// the list.
+//
+// A range's workgroup walks its cameras' active pairs alone, so few feature rows
+// are cut into shorter ranges, to occupy more CUs. Backward call at ranges of
+// 2048, 512, 256 and 128 rows: 4.7 k rows (2 x 4 cameras of 21 x 22 and 11 x 11)
+// 52, 42, 42 and 40 us; 60 k rows (2 x 2 cameras, SparseDrive's maps, 12220 pairs)
+// 89, 83, 83 and 85 us; 718 k rows (SparseDrive's batch) 485, 495, 513 and 551 us.
+//
+// A workgroup of the sums takes rows for about 96 contributions, were every pair
+// active, on average: 16 rows of small maps under many points hold thousands, and
+// the chip then waits for a few long workgroups. At 16, 8, 4, 2 and 1 rows: 2 k
+// rows that take 150 (one camera, 21 x 72 to 3 x 9, 9603 pairs) 136, 92, 65, 51 and
+// 44 us; 26 k rows that take 54 (6 x 3 cameras, 30 x 37 to 8 x 10, 6588 pairs) 93,
+// 83, 79, 81 and 93 us; SparseDrive's batch (12.5) 513, 533, 608, 731 and 986 us.
+// Past 16384 workgroups the chip is full, and more rows share a row table's load.
+struct OwnerSplit {
+  int range_rows, sum_rows;
+};
+
+OwnerSplit split_owner(const dfa::Dims &d) {
+  const int64_t rows = static_cast<int64_t>(d.batch) * d.feat;
+  const int64_t most =  // contributions to an entry's rows
+      int64_t{4} * d.anchors * d.pts * d.cams * d.scales;
+  OwnerSplit o{dfa::kRangeRows, 1};
+  while (o.range_rows > 256 && rows < int64_t{64} * o.range_rows) o.range_rows /= 2;
+  while (o.sum_rows < dfa::kSumRows &&
+         (2 * o.sum_rows * most <= int64_t{96} * d.feat || rows > int64_t{16384} * o.sum_rows)) {
+    o.sum_rows *= 2;
+  }
+  return o;
+}
+
+// Whether the sums by owner beat the atomics. They list and sum at a cost per
+// feature row and per active pair of a camera; the atomics pay per contribution,
+// and where maps are small, for adds that meet in one row. Measured as the backward
+// call with atomics over the call with owner sums (some 600 shapes of 1 to 8 entries, 1
+// to 6 cameras, 250 to 240000 pairs, most with 18.6% of the pairs active):
+// - 128 channels and more, two scales and more, up to 32768 rows a camera: 1.1 to 6
+//   (geometric mean 2.0). 64 channels: 0.7 to 2.7 (1.1).
+// - One scale: 0.4 to 2.8 (1.03): every camera's pairs are listed for a fourth of
+//   the adds.
+// - Larger maps (200 x 200 with 100 x 100, 400 x 400): few adds meet. 0.65 to 0.9 for
+//   one and two (entry, camera) pairs, whose list one workgroup writes each; from
+//   four on 0.84 to 0.96 at 1300 pairs a camera, 1.2 to 2.3 from 11700. 64 channels
+//   0.3 to 0.8.
+bool owner_is_faster(const dfa::Dims &d) {
+  if (d.scales < 2 || d.cams == 0) return false;
+  const int64_t rows = d.feat / d.cams;
+  const int64_t pairs = static_cast<int64_t>(d.anchors) * d.pts;
+  return rows <= 32768 ||
+         (d.embeds >= 128 && static_cast<int64_t>(d.batch) * d.cams >= 4 &&
+          2 * pairs * d.scales >= rows);
+}
+
 // The backward with grad_feat overwritten: feature gradients by owner sums
 // when `workspace` holds them.
 int backward_ws_impl(const char *fn, const float *feat, const int32_t *shape,
@@ -324,7 +380,9 @@ int backward_ws_impl(const char *fn, const float *feat, const int32_t *shape,
   const bool aligned = reinterpret_cast<uintptr_t>(workspace) % 256 == 0;
   if (!sampled || !plan_owner(d, w) || !workspace || workspace_bytes < w.bytes || !aligned) {
     if (n_feat > 0) {
-      dfa::dfa_zero<<<generic_blocks(n_feat), dfa::kBlock, 0, st>>>(grad_feat, n_feat);
+      const int64_t blocks = (n_feat / 4 + dfa::kBlock) / dfa::kBlock;
+      dfa::dfa_zero<<<static_cast<int>(blocks < (1 << 22) ? blocks : 1 << 22), dfa::kBlock, 0,
+                      st>>>(grad_feat, n_feat);
     }
     if (!sampled) return check_launch(fn);
     return backward_impl(fn, true, feat, shape, start, loc, weights, grad_out, grad_feat,
@@ -338,15 +396,16 @@ int backward_ws_impl(const char *fn, const float *feat, const int32_t *shape,
   dfa::Contribution *contrib = reinterpret_cast<dfa::Contribution *>(ws + w.contrib);
   const int nt = row_slots(d);
   dfa::dfa_list_active<<<d.batch * d.cams, dfa::kListBlock, 0, st>>>(loc, list, list_n, cursor, d);
-  const int ranges = (d.feat + dfa::kRangeRows - 1) / dfa::kRangeRows;
+  const OwnerSplit split = split_owner(d);
+  const int ranges = (d.feat + split.range_rows - 1) / split.range_rows;
   dfa::dfa_list_rows<<<d.batch * ranges, dfa::kRangeBlock, 0, st>>>(
-      shape, start, list, list_n, cursor, rows, contrib, d, ranges);
+      shape, start, list, list_n, cursor, rows, contrib, d, ranges, split.range_rows);
   launch_backward_rows<false>(nt, feat, shape, start, loc, weights, grad_out, nullptr, grad_loc,
                               grad_weights, d, 0, st);
-  const int per_entry = (d.feat + dfa::kSumRows - 1) / dfa::kSumRows;
+  const int per_entry = (d.feat + split.sum_rows - 1) / split.sum_rows;
   auto sum = [&](auto slots) {
     dfa::dfa_sum_rows<decltype(slots)::value><<<d.batch * per_entry, dfa::kBlock, 0, st>>>(
-        weights, grad_out, rows, contrib, grad_feat, d, per_entry);
+        weights, grad_out, rows, contrib, grad_feat, d, per_entry, split.sum_rows);
   };
   switch (nt) {
     case 1: sum(std::integral_constant<int, 1>()); break;
@@ -411,6 +470,19 @@ size_t deformable_aggregation_backward_workspace_size(int64_t batch, int64_t num
   if (validate("deformable_aggregation_backward_workspace_size", a, d) != 0) return 0;
   if (static_cast<int64_t>(d.batch) * d.anchors * d.pts * d.cams == 0) return 0;
   return plan_owner(d, w) ? w.bytes : 0;
+}
+
+int deformable_aggregation_backward_prefers_workspace(int64_t batch, int64_t num_cams,
+                                                      int64_t num_feat, int64_t num_embeds,
+                                                      int64_t num_scale, int64_t num_anchors,
+                                                      int64_t num_pts, int64_t num_groups) {
+  const DfaArgs a{batch, num_cams, num_feat, num_embeds, num_scale, num_anchors, num_pts,
+                  num_groups};
+  dfa::Dims d;
+  OwnerWorkspace w;
+  if (validate("deformable_aggregation_backward_prefers_workspace", a, d) != 0) return 0;
+  if (static_cast<int64_t>(d.batch) * d.anchors * d.pts * d.cams == 0) return 0;
+  return plan_owner(d, w) && owner_is_faster(d) ? 1 : 0;
 }
 
 int deformable_aggregation_backward_ws(

@@ -392,7 +392,7 @@ __global__ void __launch_bounds__(kBlock)
   const uint32_t batch_row = static_cast<uint32_t>(b) * static_cast<uint32_t>(d.feat);
   const uint64_t below = (uint64_t{1} << lane) - 1;
   const int sgd = sg > 0 ? sg : 1;  // no scales: nothing is zeroed
-  const int own_n = sg > 0 ? kWave / parts : 0;  // pairs of a run this part zeroes if skipped
+  const int parts_log2 = __builtin_ctz(parts);
   const int lane_i = lane / sgd, lane_j = lane - lane_i * sgd;
   const int step_i = kWave / sgd, step_j = kWave - step_i * sgd;
   int seen = 0;  // active pairs of the row before this run of 64
@@ -408,9 +408,10 @@ __global__ void __launch_bounds__(kBlock)
     // weight gradients of skipped pairs are zero: element j of this part's
     // i-th pair p = part + i * parts of the run (base is a multiple of parts),
     // (i, j) stepped by kWave elements per pass (no division inside)
+    const int own_n = sg > 0 ? (n - part + parts - 1) >> parts_log2 : 0;
     for (int i = lane_i, j = lane_j; i < own_n;) {
       const int p = part + i * parts;
-      if (p < n && !((act >> p) & 1)) gw_row[static_cast<size_t>(base + p) * sg + j] = 0.0f;
+      if (!((act >> p) & 1)) gw_row[static_cast<size_t>(base + p) * sg + j] = 0.0f;
       i += step_i;
       j += step_j;
       if (j >= sg) {
@@ -522,16 +523,17 @@ __global__ void __launch_bounds__(kBlock)
 // (row table, contributions, rows). Persistent workgroups with the tables
 // loaded blocks ahead were slower (281-301 us: a wavefront's loads then wait for
 // its earlier stores, which complete in order), and so were 32 rows a
-// workgroup (280 us) and eight rows requested at a time (273 us).
+// workgroup (280 us) and eight rows requested at a time (273 us). Smaller maps
+// and fewer points are split finer (split_owner in dfa_capi.hip).
 //
 // Sums are float64 over the exact products w_corner * (grad_out * weight), the
 // operands float32, and are rounded once, so their order (which the counting
 // sort leaves open) does not show.
 
 constexpr int kListBlock = 1024;
-constexpr int kRangeRows = 2048;  // feature rows counted by one workgroup of dfa_list_rows
+constexpr int kRangeRows = 2048;  // most feature rows counted by one workgroup of dfa_list_rows
 constexpr int kRangeBlock = 512;
-constexpr int kSumRows = 16;  // feature rows of one workgroup of dfa_sum_rows; divides kRangeRows
+constexpr int kSumRows = 16;  // most feature rows of one workgroup of dfa_sum_rows
 constexpr int kSumUnroll = 4;
 
 // One contribution to a feature row: element (pt-camera pair and scale) index of
@@ -583,7 +585,7 @@ __global__ void __launch_bounds__(kListBlock)
   if (tid == 0) list_n[blockIdx.x] = n_list;
 }
 
-// Contributions of kRangeRows feature rows of one batch entry, sorted by row.
+// Contributions of range_rows feature rows of one batch entry, sorted by row.
 // The workgroup walks the active pairs of the cameras whose maps meet its rows
 // twice: counting per row in LDS, then, with the counts scanned and its run of
 // `contrib` reserved, storing. rows[b * feat + r] = the row's [start, end) in
@@ -593,7 +595,7 @@ __global__ void __launch_bounds__(kRangeBlock)
     dfa_list_rows(const int32_t *__restrict__ shape, const int32_t *__restrict__ start,
                   const float4 *__restrict__ list, const uint32_t *__restrict__ list_n,
                   uint32_t *__restrict__ cursor, uint2 *__restrict__ rows,
-                  Contribution *__restrict__ contrib, Dims d, int ranges) {
+                  Contribution *__restrict__ contrib, Dims d, int ranges, int range_rows) {
   constexpr int kWaves = kRangeBlock / kWave;
   constexpr int kPer = kRangeRows / kRangeBlock;  // rows scanned by a thread
   __shared__ View views[kMaxViews];
@@ -603,8 +605,8 @@ __global__ void __launch_bounds__(kRangeBlock)
   stage_views(views, shape, start, d);
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   const int lb = msda::xcd_logical_block(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
-  const int b = lb / ranges, r0 = (lb % ranges) * kRangeRows;
-  const int n_rows = min(kRangeRows, d.feat - r0);
+  const int b = lb / ranges, r0 = (lb % ranges) * range_rows;
+  const int n_rows = min(range_rows, d.feat - r0);
   for (int i = tid; i < kRangeRows; i += kRangeBlock) count[i] = 0u;
   __syncthreads();
   const int pairs = d.anchors * d.pts;
@@ -663,7 +665,7 @@ __global__ void __launch_bounds__(kRangeBlock)
   });
 }
 
-// grad_feat of kSumRows consecutive feature rows per workgroup, every row
+// grad_feat of sum_rows consecutive feature rows per workgroup, every row
 // written (zero without contributions). The rows' contributions, contiguous,
 // are split evenly over the four wavefronts, so a row that takes many is
 // shared; a wavefront's sum of a row that an earlier wavefront began goes
@@ -675,7 +677,7 @@ template <int NT>
 __global__ void __launch_bounds__(kBlock)
     dfa_sum_rows(const float *__restrict__ weights, const float *__restrict__ grad_out,
                  const uint2 *__restrict__ rows, const Contribution *__restrict__ contrib,
-                 float *__restrict__ grad_feat, Dims d, int blocks_per_entry) {
+                 float *__restrict__ grad_feat, Dims d, int blocks_per_entry, int sum_rows) {
   using L = Lanes<NT>;
   constexpr int C = NT * kWave, kWaves = kBlock / kWave;
   __shared__ double head[kWaves][NT][kWave];  // sum of the row begun by an earlier wavefront
@@ -684,8 +686,8 @@ __global__ void __launch_bounds__(kBlock)
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
   const int lb = static_cast<int>(gridDim.x) - 1 -
                  msda::xcd_logical_block(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
-  const int b = lb / blocks_per_entry, r0 = (lb % blocks_per_entry) * kSumRows;
-  const int n = min(kSumRows, d.feat - r0);
+  const int b = lb / blocks_per_entry, r0 = (lb % blocks_per_entry) * sum_rows;
+  const int n = min(sum_rows, d.feat - r0);
   const size_t row0 = static_cast<size_t>(b) * d.feat + r0;
   const uint2 mine = rows[row0 + min(lane, n - 1)];  // lane i: row i's contributions
   auto lane_of = [](uint32_t v, int l) {
@@ -787,10 +789,17 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
+// n zeros at p, in 16-byte stores between its unaligned ends.
 __global__ void __launch_bounds__(kBlock) dfa_zero(float *__restrict__ p, int64_t n) {
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    p[i] = 0.0f;
+  const int64_t tid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t ahead = (16 - (reinterpret_cast<uintptr_t>(p) & 15)) / 4 % 4;
+  const int64_t head = ahead < n ? ahead : n;
+  const int64_t quads = (n - head) / 4, tail = head + 4 * quads;
+  if (tid < head) p[tid] = 0.0f;
+  if (tail + tid < n) p[tail + tid] = 0.0f;
+  float4 *q = reinterpret_cast<float4 *>(p + head);
+  for (int64_t i = tid; i < quads; i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    q[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   }
 }
 

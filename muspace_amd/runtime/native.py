@@ -140,6 +140,7 @@ _EXPORTS: dict[str, tuple[Any, list[Any]]] = {
     "deformable_aggregation_backward_opt": (_c_int, [_c_ptr] * 9 + [_c_int64] * 8 + [_c_ptr]),
     "deformable_aggregation_backward_base": (_c_int, [_c_ptr] * 9 + [_c_int64] * 8 + [_c_ptr]),
     "deformable_aggregation_backward_workspace_size": (ctypes.c_size_t, [_c_int64] * 8),
+    "deformable_aggregation_backward_prefers_workspace": (_c_int, [_c_int64] * 8),
     "deformable_aggregation_backward_ws": (
         _c_int, [_c_ptr] * 9 + [_c_int64] * 8 + [_c_ptr, ctypes.c_size_t, _c_ptr]
     ),
@@ -892,8 +893,8 @@ class NativeLibrary:
         ):
             _check(tensor, label, (torch.float32,))
             _check_shape(tensor, label, like)
-        scratch = ()
-        if with_workspace:
+        scratch = (None, 0) if with_workspace else ()
+        if with_workspace and self._raw["deformable_aggregation_backward_prefers_workspace"](*dims):
             nbytes = self._raw["deformable_aggregation_backward_workspace_size"](*dims)
             try:
                 workspace = torch.empty(nbytes, dtype=torch.uint8, device=mc_ms_feat.device)
@@ -901,7 +902,7 @@ class NativeLibrary:
             except torch.OutOfMemoryError:
                 # sized for every pair active, up to 8 GiB: the kernels with atomics
                 # need none of it
-                scratch = (None, 0)
+                pass
         self._launch(
             name, mc_ms_feat.device,
             mc_ms_feat.data_ptr(), spatial_shape.data_ptr(), scale_start_index.data_ptr(),
@@ -935,9 +936,9 @@ class NativeLibrary:
                                         sampling_location, weights, grad_output,
                                         grad_mc_ms_feat, grad_sampling_location,
                                         grad_weights) -> None:
-        """All three gradients overwritten (none needs zero-filling); the
-        scratch comes from torch's caching allocator, and a call that cannot
-        have it takes the kernels without."""
+        """All three gradients overwritten (none needs zero-filling). Where
+        scratch makes the call faster it comes from torch's caching allocator; a
+        call that cannot have it takes the kernels without."""
         self._dfa_backward("deformable_aggregation_backward_ws", mc_ms_feat, spatial_shape,
                            scale_start_index, sampling_location, weights, grad_output,
                            grad_mc_ms_feat, grad_sampling_location, grad_weights,

@@ -35,11 +35,43 @@ def _case(seed, shapes, channels, groups, anchors, batch=2, pts=3, cams=3):
     return case
 
 
-def _backward(case, grad_out, name="deformable_aggregation_backward"):
+def _dims(case):
+    """batch, cams, feat, embeds, scales, anchors, pts, groups"""
+    (batch, feat, embeds), weights = case[0].shape, case[4].shape
+    return [batch, weights[3], feat, embeds, weights[4], weights[1], weights[2], weights[5]]
+
+
+def _by_owner(case, grad_out):
+    """The sums by owner, with their workspace, also where the operator has the
+    atomic kernels for the faster ones."""
     mc, spatial, start, loc, weights = [t.to(DEV) for t in case]
-    poison = float("nan") if name == "deformable_aggregation_backward" else 0.0
-    grads = [torch.full_like(t, poison) for t in (mc, loc, weights)]
+    grad_out = grad_out.to(DEV)
+    grads = [torch.full_like(t, float("nan")) for t in (mc, loc, weights)]
+    lib, dims = load_native_module(), _dims(case)
+    size = lib.raw("deformable_aggregation_backward_workspace_size")(*dims)
+    assert size > 0
+    workspace = torch.empty(size, dtype=torch.uint8, device=DEV)
+    code = lib.raw("deformable_aggregation_backward_ws")(
+        *[t.data_ptr() for t in (mc, spatial, start, loc, weights, grad_out, *grads)], *dims,
+        workspace.data_ptr(), size, torch.cuda.current_stream().cuda_stream)
+    assert code == 0
+    return [g.cpu() for g in grads]
+
+
+def _backward(case, grad_out, name="deformable_aggregation_backward"):
+    if name == "deformable_aggregation_backward":
+        return _by_owner(case, grad_out)
+    mc, spatial, start, loc, weights = [t.to(DEV) for t in case]
+    grads = [torch.zeros_like(t) for t in (mc, loc, weights)]
     getattr(load_native_module(), name)(mc, spatial, start, loc, weights, grad_out.to(DEV), *grads)
+    return [g.cpu() for g in grads]
+
+
+def _operator_backward(case, grad_out):
+    """As the operator calls it: scratch where the library asks for it."""
+    case = [t.to(DEV) for t in case]
+    grads = [torch.full_like(case[i], float("nan")) for i in (0, 3, 4)]
+    load_native_module().deformable_aggregation_backward(*case, grad_out.to(DEV), *grads)
     return [g.cpu() for g in grads]
 
 
@@ -66,6 +98,33 @@ def _check(case, grad_out):
 def test_row_ranges_and_channel_layouts(channels, groups, shapes):
     case = _case(31, shapes, channels, groups, anchors=40)
     _check(case, torch.randn(2, 40, channels, generator=torch.Generator().manual_seed(32)))
+
+
+@gpu
+@pytest.mark.parametrize("shapes,batch,anchors", [
+    (((64, 88), (32, 44)), 2, 40),   # 42240 rows: ranges of 512; 16 rows a workgroup of the sums
+    (((100, 90), (50, 45)), 2, 40),  # 67500 rows: ranges of 1024
+    (((150, 160), (75, 80)), 2, 40),  # 180000 rows: ranges of 2048
+    (((25, 28), (13, 14)), 2, 60),   # 16 rows a workgroup of the sums, 8, 4, 2, 1
+    (((25, 28), (13, 14)), 2, 300),
+    (((25, 28), (13, 14)), 2, 500),
+    (((25, 28), (13, 14)), 2, 900),
+    (((25, 28), (13, 14)), 2, 1400),
+])
+def test_ranges_and_blocks_of_the_sums_by_shape(shapes, batch, anchors):
+    case = _case(47, shapes, 128, 8, anchors=anchors, batch=batch, pts=4)
+    _check(case, torch.randn(batch, anchors, 128, generator=torch.Generator().manual_seed(48)))
+
+
+@gpu
+@pytest.mark.parametrize("channels,shapes", [(64, ((7, 9), (3, 5))), (256, ((7, 9),))])
+def test_operator_with_and_without_scratch(channels, shapes):
+    """One scale takes the kernels with atomics."""
+    case = _case(49, shapes, channels, 8, anchors=50)
+    grad_out = torch.randn(2, 50, channels, generator=torch.Generator().manual_seed(50))
+    for g, e, atol in zip(_operator_backward(case, grad_out), _by_owner(case, grad_out),
+                          (1e-5, 1e-3, 1e-4)):
+        torch.testing.assert_close(g, e, rtol=1e-5, atol=atol)
 
 
 @gpu
@@ -167,11 +226,35 @@ def test_misaligned_or_short_workspace_is_left_alone(offset, short):
 
 
 @gpu
+@pytest.mark.parametrize("offset", [0, 1, 2, 3])
+@pytest.mark.parametrize("shapes", [((1, 1),), ((3, 5), (2, 2))])
+def test_gradient_zeroed_in_full_and_no_further(offset, shapes):
+    """Without a workspace the feature gradient is zeroed first, whatever the
+    alignment of its ends (3 channels, so its length is no multiple of four)."""
+    case = [t.to(DEV) for t in _case(51, shapes, 3, 1, anchors=7, batch=1, cams=1)]
+    grad_out = torch.randn(1, 7, 3, generator=torch.Generator().manual_seed(52)).to(DEV)
+    n = case[0].numel()
+    buffer = torch.full((n + 8,), 7.0, device=DEV)
+    rest = [torch.empty_like(case[i]) for i in (3, 4)]
+    lib = load_native_module()
+    code = lib.raw("deformable_aggregation_backward_ws")(
+        *[t.data_ptr() for t in (*case, grad_out)], buffer.data_ptr() + 4 * (offset + 4),
+        *[t.data_ptr() for t in rest], *_dims(case), None, 0,
+        torch.cuda.current_stream().cuda_stream)
+    assert code == 0
+    got, outside = buffer[offset + 4: offset + 4 + n], torch.ones(n + 8, dtype=torch.bool)
+    outside[offset + 4: offset + 4 + n] = False
+    assert (buffer.cpu()[outside] == 7.0).all()
+    base = _backward(case, grad_out, "deformable_aggregation_backward_base")
+    torch.testing.assert_close(got.cpu().view_as(base[0]), base[0], rtol=1e-5, atol=1e-5)
+
+
+@gpu
 def test_scratch_that_cannot_be_had(monkeypatch):
     """Out of memory for the scratch alone: the call takes the kernels without it."""
     case = _case(45, ((9, 13), (4, 6)), 256, 8, anchors=60)
     grad_out = torch.randn(2, 60, 256, generator=torch.Generator().manual_seed(46))
-    expected = _backward(case, grad_out)
+    expected = _operator_backward(case, grad_out)
     asked, empty = [], torch.empty
 
     def no_bytes(*args, **kwargs):
@@ -181,7 +264,7 @@ def test_scratch_that_cannot_be_had(monkeypatch):
         return empty(*args, **kwargs)
 
     monkeypatch.setattr(torch, "empty", no_bytes)
-    actual = _backward(case, grad_out)
+    actual = _operator_backward(case, grad_out)
     assert asked
     for a, e, atol in zip(actual, expected, (1e-5, 1e-3, 1e-4)):
         torch.testing.assert_close(a, e, rtol=1e-5, atol=atol)
@@ -201,3 +284,22 @@ def test_workspace_size_and_validation(native_lib):
     assert "null tensor pointer" in native_lib.last_error()
     assert fn(*[1] * 9, *dims[:7], 9, None, 0, None) == 1
     assert "num_groups must be in [1, 8]" in native_lib.last_error()
+
+
+@pytest.mark.parametrize("dims,owner", [
+    # batch, cams, feat, embeds, scales, anchors, pts, groups
+    ([8, 6, 89760, 256, 4, 900, 13, 8], True),    # SparseDrive's batch
+    ([1, 1, 500, 128, 2, 50, 5, 8], True),        # the smallest maps and fewest points
+    ([1, 1, 500, 64, 2, 50, 5, 8], True),
+    ([2, 6, 60000, 128, 1, 1227, 5, 8], False),   # one scale
+    ([1, 1, 32768, 256, 2, 900, 13, 8], True),    # 32768 rows a camera ...
+    ([1, 1, 32769, 256, 2, 900, 13, 8], False),   # ... more, and one (entry, camera)
+    ([4, 1, 50000, 256, 2, 12500, 1, 8], True),   # four of them, and many pairs
+    ([4, 1, 50000, 256, 2, 12499, 1, 8], False),
+    ([3, 1, 50000, 256, 2, 12500, 1, 8], False),
+    ([4, 1, 50000, 64, 2, 12500, 1, 8], False),   # 64 channels
+    ([1, 1, 500, 96, 2, 50, 5, 8], False),        # no row kernel
+    ([1, 1, 500, 128, 2, 0, 5, 8], False),        # nothing sampled
+])
+def test_which_shapes_take_the_sums_by_owner(native_lib, dims, owner):
+    assert native_lib.raw("deformable_aggregation_backward_prefers_workspace")(*dims) == owner
