@@ -133,12 +133,24 @@ void launch_coarse(const int32_t *shape, const int32_t *start, const float *loc,
       shape, start, loc, weights, grad_out, grad_feat, d, budget, pair_log2, ns);
 }
 
-// Wavefronts per row of dfa_forward_rows: few rows give each of the 1024 SIMDs
-// few wavefronts with long serial pair walks, so a row's pairs are shared.
-// SparseDrive's 900 rows of one sample: 37.1, 31.2, 30.5 and 29.9 us at 2, 4, 8
-// and 16; its batch of 7,200 rows: 194.9, 185.8, 182.6 and 185.9 us.
-int forward_parts(int rows) {
-  return rows >= 8192 * 4 ? 1 : rows >= 8192 * 2 ? 2 : rows >= 2048 ? 8 : 16;
+// Wavefronts per row of dfa_forward_rows (a power of two up to 16). Few rows give
+// each of the 1024 SIMDs few wavefronts with long serial pair walks, so a row's
+// pairs are shared, until there are about 8192 wavefronts: from there on each one's
+// own cost (maps, locations, its part of the sum) grows the total. At 4, 8 and 16,
+// 78 pairs a row: 300 rows of 256 channels 17.1, 14.6 and 15.0 us (64 channels: 11.4,
+// 8.8, 8.7); 900 rows 29.4, 28.4, 28.6 (15.6, 13.3, 15.3); 1800 rows of 64 channels
+// 20.3, 20.6 and 24.9, of 128 27.5, 26.4 and 28.9. Long rows of 192 and 256 channels
+// hold enough work for 8: 1800 rows 53.5 us at 4, 50.6 at 8; 7200 rows 184 and 179;
+// but 1970 rows of 18 pairs 10.6 and 12.2. From 16384 rows on two wavefronts, from
+// 32768 one (24000 rows of 64 channels: 160 us at 2, 166 at 4).
+int forward_parts(const dfa::Dims &d) {
+  const int rows = d.batch * d.anchors;
+  if (rows >= 8192 * 4) return 1;
+  if (rows >= 8192 * 2) return 2;
+  int parts = 4;
+  while (parts < 16 && rows <= 8192 / (2 * parts)) parts *= 2;
+  if (parts == 4 && d.embeds >= 192 && d.pts * d.cams >= 64) parts = 8;
+  return parts;
 }
 
 int forward_impl(const char *fn, bool optimized, const float *feat, const int32_t *shape,
@@ -154,7 +166,7 @@ int forward_impl(const char *fn, bool optimized, const float *feat, const int32_
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int nt = optimized ? row_slots(d) : 0;
   const int rows = d.batch * d.anchors;
-  const int parts = forward_parts(rows);
+  const int parts = forward_parts(d);
   const int block = parts * dfa::kWave > dfa::kBlock ? parts * dfa::kWave : dfa::kBlock;
   const int per_block = block / dfa::kWave;
   const int blocks = (rows * parts + per_block - 1) / per_block;

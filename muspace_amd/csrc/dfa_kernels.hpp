@@ -224,25 +224,27 @@ struct Lanes {
   }
 };
 
-// A pair's corner rows and weights are loaded kScaleRun scales at a time before
-// either is used, so one memory latency covers them.
+// The backward loads a pair's corner rows and weights kScaleRun scales at a time
+// before either is used, so one memory latency covers them (the forward's loop is
+// unrolled as far).
 constexpr int kScaleRun = 2;
 constexpr int kMaxParts = 16;  // wavefronts per (batch, anchor) row
 
-// The loads of one run of scales of one pair at (x, y): corner rows (zeros
-// outside the map and for scales past the last) and the lane's weights.
+// The taps of one run of scales of one pair at (x, y), and its loads: corner rows
+// (zeros outside the map and for scales past the last) and the lane's weights. The
+// taps are kept: in rows of 64 channels their arithmetic is a third of the work.
 template <int NT, typename L>
 __device__ __forceinline__ void load_run(__amdgpu_buffer_rsrc_t rf, uint32_t batch_row,
                                          const View *cv, const float *wp, const int (&grp)[NT],
                                          float x, float y, int s0, int lane, const Dims &d,
-                                         float (&val)[kScaleRun][4][NT],
+                                         Tap (&taps)[kScaleRun], float (&val)[kScaleRun][4][NT],
                                          float (&wv)[kScaleRun][L::kGroups]) {
   constexpr int C = NT * kWave;
 #pragma unroll
   for (int j = 0; j < kScaleRun; ++j) {
     const int s = min(s0 + j, d.scales - 1);
     const View v = cv[s];
-    const Tap tp = make_tap(x, y, v);
+    const Tap &tp = taps[j] = make_tap(x, y, v);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const bool ok = s0 + j < d.scales && v.h > 0 && tp.cell[k] >= 0;
@@ -258,14 +260,16 @@ __device__ __forceinline__ void load_run(__amdgpu_buffer_rsrc_t rf, uint32_t bat
 // Forward, one (batch, anchor) row over `parts` (a power of two up to 16)
 // wavefronts of one workgroup: the row's active pairs are dealt round-robin by
 // their rank among the active pairs, and the parts' partial rows are summed
-// through LDS by part 0, which adds the row to `out`.
+// through LDS by part 0, which adds the row to `out`. Only rows of 256 channels
+// take packed lanes (8 x 3000 rows of 128 in 8-byte loads: 258 us, in two 4-byte
+// loads 249).
 template <int NT>
 __global__ void __launch_bounds__(kMaxParts * kWave)
     dfa_forward_rows(const float *__restrict__ feat, uint32_t feat_bytes,
                      const int32_t *__restrict__ shape, const int32_t *__restrict__ start,
                      const float *__restrict__ loc, const float *__restrict__ weights,
                      float *__restrict__ out, Dims d, int parts) {
-  using L = Lanes<NT>;
+  using L = Lanes<NT, NT == 4>;
   constexpr int C = NT * kWave;
   __shared__ View views[kMaxViews];
   extern __shared__ float partial[];  // [wavefronts][C] when parts > 1
@@ -307,18 +311,24 @@ __global__ void __launch_bounds__(kMaxParts * kWave)
       const int pair = base + l, cam = pair % d.cams;
       const float *wp = w_row + static_cast<size_t>(pair) * sg;
       const View *cv = views + cam * d.scales;
-      for (int s0 = 0; s0 < d.scales; s0 += kScaleRun) {
-        float val[kScaleRun][4][NT], wv[kScaleRun][L::kGroups];
-        load_run<NT, L>(rf, batch_row, cv, wp, grp, x, y, s0, lane, d, val, wv);
+#pragma unroll 2
+      for (int s = 0; s < d.scales; ++s) {
+        const View v = cv[s];
+        const Tap tp = make_tap(x, y, v);
+        float val[4][NT], wv[L::kGroups];
 #pragma unroll
-        for (int j = 0; j < kScaleRun; ++j) {
-          if (s0 + j >= d.scales) break;  // uniform
-          const Tap tp = make_tap(x, y, cv[s0 + j]);
+        for (int k = 0; k < 4; ++k) {
+          const bool ok = v.h > 0 && tp.cell[k] >= 0;
+          L::gather(
+              rf, ok ? (batch_row + static_cast<uint32_t>(v.start + tp.cell[k])) * (C * 4u) : kOobOffset,
+              lane, val[k]);
+        }
 #pragma unroll
-          for (int t = 0; t < NT; ++t) {
-            acc[t] += (tp.w[0] * val[j][0][t] + tp.w[1] * val[j][1][t] + tp.w[2] * val[j][2][t] +
-                       tp.w[3] * val[j][3][t]) * wv[j][L::kPacked ? 0 : t];
-          }
+        for (int t = 0; t < L::kGroups; ++t) wv[t] = wp[s * d.groups + grp[t]];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          acc[t] += (tp.w[0] * val[0][t] + tp.w[1] * val[1][t] + tp.w[2] * val[2][t] +
+                     tp.w[3] * val[3][t]) * wv[L::kPacked ? 0 : t];
         }
       }
     }
@@ -432,14 +442,15 @@ __global__ void __launch_bounds__(kBlock)
       const View *cv = views + cam * d.scales;
       float gx = 0.0f, gy = 0.0f;
       for (int s0 = 0; s0 < d.scales; s0 += kScaleRun) {
+        Tap taps[kScaleRun];
         float val[kScaleRun][4][NT], wv[kScaleRun][L::kGroups];
-        load_run<NT, L>(rf, batch_row, cv, wp, grp, x, y, s0, lane, d, val, wv);
+        load_run<NT, L>(rf, batch_row, cv, wp, grp, x, y, s0, lane, d, taps, val, wv);
 #pragma unroll
         for (int j = 0; j < kScaleRun; ++j) {
           const int s = s0 + j;
           if (s >= d.scales) break;  // uniform
           const View v = cv[s];
-          const Tap tp = make_tap(x, y, v);
+          const Tap &tp = taps[j];
           float gwt[L::kGroups];
           // per weight the lane holds, g times the sample and its slopes, summed
           // over the channels under that weight (all the lane's, or one)

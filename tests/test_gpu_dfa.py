@@ -416,3 +416,19 @@ def test_random_shapes_backward_matches_the_oracle(seed):
     torch.testing.assert_close(gf.cpu().double(), ef, rtol=1e-4, atol=1e-4 * scale)
     torch.testing.assert_close(gl.cpu().double(), el, rtol=1e-4, atol=1e-3 * scale)
     torch.testing.assert_close(gw.cpu().double(), ew, rtol=1e-4, atol=1e-4 * scale)
+
+
+# wavefronts per row of the forward: 16 to 512 rows, 8 to 1024, 4 from there (8 for
+# long rows of 192 channels and more), at one and at many pairs a row
+# (sums of up to 66 pairs x 3 maps x 4 corners, products around 1: 800 * 2^-24 = 5e-5)
+@pytest.mark.parametrize("channels,groups", [(64, 8), (128, 4), (192, 3), (256, 8)])
+@pytest.mark.parametrize("rows,pts,cams", [(1, 1, 1), (512, 3, 2), (513, 3, 2), (1024, 2, 3),
+                                           (1025, 3, 2), (1025, 11, 6), (1030, 13, 5)])
+def test_forward_wavefronts_per_row(channels, groups, rows, pts, cams):
+    case = random_case(71, batch=1, anchors=rows, pts=pts, cams=cams, channels=channels,
+                       groups=groups, shapes=((6, 7), (3, 4), (2, 2)), dtype=torch.float32,
+                       boundary=pts > 1)
+    out = torch.ones((1, rows, channels), device=DEV)
+    load_native_module().deformable_aggregation_forward_opt(*[t.to(DEV) for t in case], out)
+    ref = dfa_torch.aggregate_batched(*[t.double() if t.is_floating_point() else t for t in case])
+    torch.testing.assert_close(out.cpu().double(), 1 + ref, rtol=1e-5, atol=1e-4)
