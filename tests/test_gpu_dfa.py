@@ -432,3 +432,18 @@ def test_forward_wavefronts_per_row(channels, groups, rows, pts, cams):
     load_native_module().deformable_aggregation_forward_opt(*[t.to(DEV) for t in case], out)
     ref = dfa_torch.aggregate_batched(*[t.double() if t.is_floating_point() else t for t in case])
     torch.testing.assert_close(out.cpu().double(), 1 + ref, rtol=1e-5, atol=1e-4)
+
+
+def test_partial_rows_of_the_forward_are_summed_pairwise():
+    """A row's 78 pairs are summed by 16 wavefronts, and the partial sums as a tree:
+    the relative error against 64 bits measures 9.3e-8 to 9.4e-8 (three seeds); the
+    partial rows added one after another, 1.07e-7 to 1.08e-7."""
+    case = list(random_case(61, batch=2, anchors=64, pts=13, cams=6,
+                            shapes=((32, 64), (16, 32), (8, 16), (4, 8)), channels=256, groups=8,
+                            dtype=torch.float32))
+    case[3].copy_(torch.round(case[3] * 4096) / 4096)  # float32 cell coordinates are exact
+    case = [t.to(DEV) for t in case]
+    out = torch.zeros((2, 64, 256), device=DEV)
+    load_native_module().deformable_aggregation_forward_opt(*case, out)
+    ref = dfa_torch.aggregate_batched(*[t.double() if t.is_floating_point() else t for t in case])
+    assert (out.double() - ref).norm() <= 1.0e-7 * ref.norm()
