@@ -427,6 +427,26 @@ def test_value_past_2gib_takes_the_wide_paths(native_lib, path):
         _assert_close(ga[sl], o_ga, 1e-4, f"grad_attention_weights[{b}]")
 
 
+@pytest.mark.parametrize("path", ["one_call", "fused"])
+@pytest.mark.parametrize("levels", [((200, 200), (100, 95)), ((200, 200), (100, 100)),
+                                    ((206, 206), (103, 100)), ((215, 215), (107, 100))])
+def test_lds_near_the_default_limit(native_lib, levels, path):
+    """Tile tables of 3810 to 4381 entries: bin_scatter's dynamic LDS is just below and above
+    64 KB, and its static tables come on top."""
+    t, grad = small_case(23, 1, 300, 2, 32, levels, 4)
+    if path == "fused":
+        out, gv, gl, ga = run_fused(native_lib, t, grad, torch.float32, torch.float32)
+        e_out = msda_torch.msda_forward(*oracle_inputs(t, torch.float32, torch.float32))
+        _assert_close(out, e_out, 1e-5, "output")
+    else:
+        gv, gl, ga = run_backward(native_lib, t, grad, torch.float32, torch.float32)
+    value, shapes, loc, attn = oracle_inputs(t, torch.float32, torch.float32)
+    _, e_gv, e_gl, e_ga = msda_torch.msda_forward_backward(value, shapes, loc, attn, grad)
+    _assert_close(gv, e_gv, 1e-4, "grad_value")
+    _assert_close(gl, e_gl, 1e-4, "grad_sampling_locations")
+    _assert_close(ga, e_ga, 1e-4, "grad_attention_weights")
+
+
 @pytest.mark.parametrize("value_dtype", [torch.float32, torch.bfloat16])
 def test_half_pixel_known_answer_2048(native_lib, value_dtype):
     """Reference KAT (tests/ops/test_multi_scale_deformable_attn.py:430-468)."""
