@@ -60,7 +60,11 @@ namespace msda {
 // spill to scratch).
 constexpr int kTileBlock = 768;
 constexpr int kBinBlock = 256;           // binning workgroup
-constexpr int kMaxTilesPerSlab = 16384;  // LDS histogram of the binning kernels
+// Tiles of a slab and sample slots of a query that are binned; shapes past either
+// take the atomic kernels. The binning kernels' LDS tables hold them (checked at
+// bin_scatter, whose tables are the largest).
+constexpr int kMaxTilesPerSlab = 14847;
+constexpr int kMaxBinnedSamples = 2048;
 constexpr int kZeroList = 2048;          // tiles listed for zeroing per slab
 constexpr size_t kTileLdsLimit = 160 * 1024;
 constexpr int kXcdQueues = 8;            // item queues of the tile kernel (one per XCD)
@@ -583,6 +587,10 @@ __host__ __device__ constexpr size_t scatter_lds_bytes(int tile_bound) {
          static_cast<size_t>(tile_bound + 1) * 4 +              // write cursors
          (static_cast<size_t>(tile_bound + 2) / 2 * 4);         // 16-bit counts, then offsets
 }
+
+static_assert(scatter_lds_bytes(kMaxTilesPerSlab) + 4096 <= kTileLdsLimit, "bin_scatter LDS");
+static_assert(kMaxBinnedSamples <= kScatterSlots, "a sub-chunk holds a query's samples");
+static_assert(kMaxTilesPerSlab < 65535, "16-bit tile numbers");
 
 // Writes each sample's 16-byte record into its tile's range and its record
 // index into the sample -> record map. A sub-chunk's records are ranked per

@@ -531,7 +531,8 @@ void launch_scatter_div(const void *value, const int64_t *shapes, const int64_t 
       }
     }
     forward_rows_ns<VT, C>(s, [&](auto ns, const Launch &L) {
-      // one segment of whole blocks per camera (the plan depends on L*P only)
+      // one segment of whole blocks per camera; the plan's units per lane group come
+      // from all cameras' units together, the same for every segment
       msda::CameraSlots<VT, GT, kAtomic> seg = out;
       const int64_t per_wave = static_cast<int64_t>((msda::kWave / KQ) >> L.plan.gu_log2) *
                                L.plan.iters;
@@ -810,10 +811,8 @@ bool plan_tile_workspace(const msda::Shape &s, int value_dtype, TileWorkspace &w
   const int64_t bound = static_cast<int64_t>(s.spatial) / T + s.levels + 1;
   if (bound > msda::kMaxTilesPerSlab) return false;
   p.tile_bound = static_cast<int>(bound);
-  // the binning kernels' LDS tables of a word per tile (bin_count's the largest)
-  if (bound > 14847) return false;
   p.lp_log2 = log2_int(s.lp > 0 ? s.lp : 1);
-  if ((1 << p.lp_log2) > 2048) return false;
+  if ((1 << p.lp_log2) > msda::kMaxBinnedSamples) return false;
   // record ids pack (q << lp_log2) | sample below bit kPosShift and the tap's
   // position in the tile frame above it
   if ((static_cast<int64_t>(s.queries) << p.lp_log2) > (int64_t{1} << msda::kPosShift)) return false;

@@ -45,3 +45,15 @@ def test_channels_without_a_tile_path_do_not_fuse(native_lib, channels):
     value = torch.empty((2, 300, 4, channels), device="meta")
     loc = torch.empty((2, 200, 4, 2, 4, 2), device="meta")
     assert not native_lib.forward_bin_fuses(value, loc)
+
+
+@pytest.mark.parametrize("cells,queries,levels,points,binned", [
+    (192959, 100, 3, 4, True),   # 14843 tiles of 13 cells, and one a level and one more
+    (192985, 100, 3, 4, False),  # 14845, so past 14847 with those
+    (4000, 100, 1, 2048, True),  # 2048 sample slots a query
+    (4000, 100, 1, 2049, False),
+])
+def test_limits_of_the_binned_backward(native_lib, cells, queries, levels, points, binned):
+    value = torch.empty((1, cells, 1, 32), device="meta")
+    loc = torch.empty((1, queries, 1, levels, points, 2), device="meta")
+    assert (native_lib.backward_workspace_bytes(value, loc) > 0) == binned
