@@ -191,6 +191,16 @@ MUSPACE_API int ms_deform_attn_forward_bin(
     int64_t num_query, int64_t num_point, int64_t im2col_step, void *workspace,
     size_t workspace_bytes, void *stream);
 
+/* 1 if ms_deform_attn_forward, given 16-byte-aligned value and output, works on a
+ * slab (one batch entry and head) per workgroup for these dims, the coarse levels
+ * in LDS; 0 for the kernels that gather every row from memory. num_cams > 0 asks
+ * the same of ms_deform_attn_forward_scatter_div_cams with cameras of num_query
+ * valid rows at most. Results are the same either way. No reference counterpart. */
+MUSPACE_API int ms_deform_attn_forward_slab(int value_dtype, int64_t num_cams, int64_t batch,
+                                            int64_t spatial_size, int64_t num_heads,
+                                            int64_t channels, int64_t num_levels,
+                                            int64_t num_query, int64_t num_point);
+
 /* 1 if the forward kernel of ms_deform_attn_forward_bin, given 16-byte-aligned
  * tensors and a 256-byte-aligned workspace of
  * ms_deform_attn_backward_workspace_size bytes, can store the backward's

@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <climits>
+#include <cmath>
 #include <cstdint>
 #include <initializer_list>
 #include <mutex>
@@ -236,11 +237,31 @@ struct SlabLaunch {
   bool ok = false;
   bool narrow = false;  // 4 wavefronts a workgroup, two workgroups a CU
   bool wide = false;    // several samples per geometry load
+  bool coarse = false;  // a level in LDS, if the levels are a pyramid
+  bool ragged = false;  // the row kernel's steps are less than 9/10 full
   msda::SlabPlan plan{};
 };
 
 int slab_chunks(const SlabLaunch &L, int queries) {
   return (queries + L.plan.chunk_q - 1) / L.plan.chunk_q;
+}
+
+// Cells that the slab kernel holds in LDS (workgroups of eight wavefronts).
+int slab_cells(const msda::Shape &s, size_t elem) {
+  if (elem == 4) {
+    return s.channels == 32 ? msda::SlabCfg<float, 32, 8>::kCells
+                            : msda::SlabCfg<float, 64, 8>::kCells;
+  }
+  return s.channels == 32 ? msda::SlabCfg<__half, 32, 8>::kCells
+                          : msda::SlabCfg<__half, 64, 8>::kCells;
+}
+
+// Share of the forward row kernel's sample slots that hold one of a unit's L*P.
+double row_fill(const msda::Shape &s, size_t elem) {
+  const int kq = static_cast<int>(s.channels * elem) / 16;
+  const Launch L = plan_rows(s, kq, elem == 2 && s.channels >= 64 ? 4 : 8, true);
+  const int step = L.ns << L.plan.gu_log2;
+  return static_cast<double>(s.lp) / ((s.lp + step - 1) / step * step);
 }
 
 // Whether a forward over `slabs` slabs of `queries` queries (for cameras: the
@@ -252,28 +273,74 @@ int slab_chunks(const SlabLaunch &L, int queries) {
 // 64 bytes), 16 keep it on two heads' slabs. At the SCA shape fp32 took 579, 412,
 // 325 and 385 us at 8, 16, 32 and 48 chunks, bf16 227, 275 and 309 at 16, 32 and
 // 48; 3 x 8 slabs of 10007 fp16 queries 60 us at 16 (a round and a half), 54 at
-// 20. A workgroup copies the coarse levels (up to 119 KB) first, which 4096
-// samples and more pay for (the smallest measured have 5700).
+// 20. A workgroup copies the coarse levels (up to 119 KB) first, which takes 4096
+// samples to pay for. With one level there is nothing to copy, and workgroups of
+// four wavefronts and about 2048 of them are best (200 x 200 cells, 2 x 40000
+// queries, fp32: 83 us; eight wavefronts: 112, 94 and 88 us at 32, 48 and 64
+// chunks).
 //
-// With one level there is nothing to copy, and workgroups of four wavefronts and
-// about 2048 of them are best (200 x 200 cells, 2 x 40000 queries, fp32: 83 us;
-// eight wavefronts: 112, 94 and 88 us at 32, 48 and 64 chunks).
-SlabLaunch plan_slab(const msda::Shape &s, int64_t slabs, int queries, size_t elem) {
+// Against the row kernel the slab kernel wins or loses by how full its last round
+// of queries is and how full either kernel's steps over a unit's samples are, and
+// where its chunks spread an XCD over more slabs than the L2 holds, which the row
+// kernel's consecutive units do not. 716 drawn shapes that hold the sample
+// thresholds were 0.71 to 2.5 times as fast as with the row kernel, 45 of them
+// below 0.98; of the 565 that also pass the tests below one is (0.96; geometric
+// mean 1.40), and the others would gain 1.09 on average. Whether a level is in LDS
+// decides less: without one, 2 x 20000 queries on 200 x 200 and 100 x 100 (fp32, 4
+// points) take 89 us against 104.
+//
+// Cameras take it with a level in LDS or ragged float32 steps only (six cameras of
+// 10000 rows on 200 x 200 and 100 x 100, fp32, 8 points: 285 us against 266). In
+// 16 bits each camera is a launch, with which the row kernel fills less of the
+// chip, so the slab kernel needs less to win. With one level cameras keep the row
+// kernel (eight wavefronts: 158 against 130 us for 5625 rows, bf16 746 against 613
+// for 4 x 6 cameras of 10000; four wavefronts 0.98 to 1.05 of its speed). Of 150
+// drawn camera averages 18 lost, down to 0.82; the 116 that pass here are 0.97 to
+// 1.95 times as fast (1.31), the others 0.99 on average.
+SlabLaunch plan_slab(const msda::Shape &s, int64_t slabs, int queries, size_t elem,
+                     bool cameras = false) {
   SlabLaunch L;
-  if (s.lp < 4 || slabs <= 0 || queries <= 0) return L;
+  if ((s.channels != 32 && s.channels != 64) || s.lp < 4 || slabs <= 0 || queries <= 0) return L;
   L.narrow = s.levels == 1;
   const int64_t cus = 256;
-  const int64_t per_slab = s.channels * elem >= 128 ? 32 : 16;
+  const int row = static_cast<int>(s.channels * elem);  // bytes
+  const int64_t per_slab = row >= 128 ? 32 : 16;
   int64_t rounds = L.narrow ? 8 : (slabs * per_slab + cus / 2) / cus;
   if (rounds < 1) rounds = 1;
   int64_t chunks = cus * rounds / slabs;
   if (chunks < 1) chunks = 1;
   L.plan.chunk_q = static_cast<int>((queries + chunks - 1) / chunks);
-  L.ok = static_cast<int64_t>(L.plan.chunk_q) * s.lp >= (L.narrow ? 1024 : 4096);
+  chunks = slab_chunks(L, queries);
+  const int64_t samples = static_cast<int64_t>(L.plan.chunk_q) * s.lp;
+  const int64_t lines = static_cast<int64_t>(s.spatial) * (row < 128 ? 128 : row);
+  if (L.narrow) {
+    // fewer than 64 chunks spread an XCD's 64 workgroups over several slabs
+    L.ok = !cameras && samples >= 1024 && (chunks >= 64 || lines <= 3700000);
+    return L;
+  }
+  if (samples < 4096) return L;
   // wide loads where every block of NS * EP = 16 samples is whole and a pair of
   // samples seldom straddles two levels (at 16 samples of 4 points: 109 against
   // 99 us)
   L.wide = s.lp >= 32 && s.lp % 16 == 0;
+  const double cells = s.spatial * 3.0 / (std::pow(4.0, s.levels) - 1.0);  // the coarsest level's
+  L.coarse = cells <= slab_cells(s, elem);
+  const double rows_full = row_fill(s, elem);
+  L.ragged = rows_full < 0.9;
+  // the share of its queries' places that a chunk fills, and of its samples'
+  const int kq = row / 16, ns = kq < 8 ? kq : 8, round = 8 * (msda::kWave / kq);
+  const int places = (L.plan.chunk_q + round - 1) / round * round;
+  const double queries_full = static_cast<double>(L.plan.chunk_q) / places;
+  const double samples_full = static_cast<double>(s.lp) / ((s.lp + ns - 1) / ns * ns);
+  const double score = queries_full * queries_full * samples_full / rows_full;
+  if (cameras && elem == 2) {
+    L.ok = score >= 0.5 && L.coarse;
+    return L;
+  }
+  L.ok = score >= (elem == 2 ? 0.74 : 0.5) &&
+         (chunks == per_slab || lines <= (elem == 2 ? 2000000 : 4200000) ||
+          (chunks % per_slab == 0 && lines <= 4200000)) &&
+         (!cameras || L.coarse || L.ragged);
   return L;
 }
 
@@ -289,7 +356,7 @@ void launch_slab(const VT *v, uint32_t vbytes, const int64_t *shapes, const int6
     k<<<blocks, Cfg::kBlock, Cfg::kLds, st>>>(v, vbytes, shapes, starts, lc, aw, out, s, L.plan);
   };
   using One = std::integral_constant<int, 1>;
-  if constexpr (std::is_same<Out, msda::DenseRows<VT>>::value) {
+  if constexpr (std::is_same<Out, msda::DenseRows<VT>>::value) {  // cameras are never narrow
     if (L.narrow) {
       go(std::integral_constant<int, 4>(), One());
       return;
@@ -516,7 +583,7 @@ void launch_scatter_div(const void *value, const int64_t *shapes, const int64_t 
         longest = len > longest ? len : longest;
       }
       const int64_t slabs = static_cast<int64_t>(s.batch) * s.heads;
-      const SlabLaunch L = plan_slab(s, slabs * out.ncam, longest, sizeof(VT));
+      const SlabLaunch L = plan_slab(s, slabs * out.ncam, longest, sizeof(VT), true);
       if (L.ok) {
         msda::CameraSlots<VT, GT, kAtomic> seg = out;
         int64_t blocks = 0;
@@ -971,15 +1038,26 @@ bool fwd_bin_fuses(const msda::Shape &s, int value_dtype, const TileWorkspace &w
 // Whether a forward with binning runs the slab forward and the binning kernels
 // although the row kernel could store the records itself. Both forms, forward
 // call and tile kernel together: encoder 2 x 22223 queries, 16 samples fp32 405 ->
-// 383 us; one 200 x 200 level fp32 300 -> 293 us; SCA 12 x 15000 queries, 32
-// samples bf16 2804 -> 2675 us. At 6 x 10000 queries, 32 samples fp32 they are
-// within 1%, and the row kernel stays there: with uniform locations a workgroup's
-// records of a fine tile are short runs, which the binning kernels' scatter pays
-// more for (159 us), and in fp32 only the smallest level fits the LDS.
+// 383 us; SCA 12 x 15000 queries, 32 samples bf16 2804 -> 2675 us. At 6 x 10000
+// queries, 32 samples fp32 they are within 1%, and the row kernel stays there (with
+// uniform locations a workgroup's records of a fine tile are short runs, which the
+// binning kernels' scatter pays more for: 159 us).
+//
+// The slab forward has to win by more than the scatter costs: with a level in LDS,
+// or against ragged steps of the row kernel in float32 (586 drawn shapes: 67 below
+// 0.98 where only plan_slab decides, down to 0.88; with this rule 5 of 375, the lowest
+// 0.96, geometric mean 1.09). One level: float32 from 80 chunks of 1200 samples on
+// (27 drawn shapes 1.00 to 1.16; BEVFormer's 200 x 200, 2 x 40000 queries, 298 -> 291
+// us), while fewer chunks reach 0.92 and 16 bits 0.98 on average.
 bool bins_apart(const msda::Shape &s, size_t elem) {
-  if (s.channels != 32 && s.channels != 64) return false;
   if (elem == 4 && s.lp >= 32) return false;
-  return plan_slab(s, static_cast<int64_t>(s.batch) * s.heads, s.queries, elem).ok;
+  const SlabLaunch L =
+      plan_slab(s, static_cast<int64_t>(s.batch) * s.heads, s.queries, elem);
+  if (!L.ok) return false;
+  if (L.narrow) {
+    return elem == 4 && slab_chunks(L, s.queries) >= 80 && L.plan.chunk_q * s.lp >= 1200;
+  }
+  return L.coarse || (elem == 4 && L.ragged);
 }
 
 // The forward with the backward's binning fused in (msda_forward_bin.hpp):
@@ -1451,6 +1529,27 @@ size_t ms_deform_attn_backward_workspace_size(int value_dtype, int64_t batch,
   TileWorkspace w;
   if (!needs_data(s) || s.lp == 0 || !plan_tile_workspace(s, value_dtype, w)) return 0;
   return w.bytes;
+}
+
+int ms_deform_attn_forward_slab(int value_dtype, int64_t num_cams, int64_t batch,
+                                int64_t spatial_size, int64_t num_heads, int64_t channels,
+                                int64_t num_levels, int64_t num_query, int64_t num_point) {
+  const Args a{batch, spatial_size, num_heads, channels, num_levels, num_query, num_point,
+               batch > 0 ? batch : 1};
+  msda::Shape s;
+  if (validate("ms_deform_attn_forward_slab", a, value_dtype, value_dtype, s)) return 0;
+  ok();
+  const size_t elem = value_dtype == MUSPACE_DTYPE_F32 ? 4 : 2;
+  int64_t slabs = batch * num_heads;
+  size_t bytes = value_bytes(s, elem);
+  if (num_cams > 0) {
+    if (elem == 4) slabs *= num_cams < msda::kMaxCams ? num_cams : msda::kMaxCams;
+    bytes *= static_cast<size_t>(num_cams);
+  }
+  return needs_data(s) && bytes + 64 <= msda::kOobOffset &&
+                 plan_slab(s, slabs, s.queries, elem, num_cams > 0).ok
+             ? 1
+             : 0;
 }
 
 int ms_deform_attn_forward_bin_fused(int value_dtype, int64_t batch, int64_t spatial_size,

@@ -65,6 +65,7 @@ _EXPORTS: dict[str, tuple[Any, list[Any]]] = {
         + [_c_ptr],
     ),
     "ms_deform_attn_backward_workspace_size": (ctypes.c_size_t, [_c_int] + [_c_int64] * 7),
+    "ms_deform_attn_forward_slab": (_c_int, [_c_int] + [_c_int64] * 8),
     "ms_deform_attn_forward_bin_fused": (_c_int, [_c_int] + [_c_int64] * 7),
     "ms_deform_attn_backward_bin": (
         _c_int,
@@ -275,6 +276,7 @@ class NativeLibrary:
             "ms_deform_attn_backward_bin": self.ms_deform_attn_backward_bin,
             "ms_deform_attn_backward_rest": self.ms_deform_attn_backward_rest,
             "ms_deform_attn_forward_bin": self.ms_deform_attn_forward_bin,
+            "forward_takes_slab": self.forward_takes_slab,
             "forward_bin_fuses": self.forward_bin_fuses,
             "ms_deform_attn_forward_softmax": self.ms_deform_attn_forward_softmax,
             "ms_deform_attn_backward_softmax": self.ms_deform_attn_backward_softmax,
@@ -517,6 +519,16 @@ class NativeLibrary:
     def backward_softmax_workspace_bytes(self, value, sampling_locations) -> int:
         """Scratch bytes of the softmax backward for these shapes."""
         return self._workspace_bytes(value, sampling_locations, softmax=True)
+
+    def forward_takes_slab(self, value, sampling_locations, num_cams: int = 0) -> bool:
+        """Whether :meth:`ms_deform_attn_forward` (``num_cams``: the camera average,
+        ``value`` of one camera) keeps a slab's coarse levels in LDS for these shapes
+        (same results either way)."""
+        batch, spatial, heads, channels = value.shape
+        _, queries, _, levels, points, _ = sampling_locations.shape
+        return bool(self._raw["ms_deform_attn_forward_slab"](
+            _dtype_code(value.dtype), num_cams, batch, spatial, heads, channels, levels, queries,
+            points))
 
     def forward_bin_fuses(self, value, sampling_locations) -> bool:
         """Whether the forward kernel of :meth:`ms_deform_attn_forward_bin` can

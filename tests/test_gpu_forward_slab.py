@@ -17,6 +17,7 @@ from conftest import gpu_available
 from muspace_amd import multi_scale_deformable_attn
 from muspace_amd.ops.msda_softmax import multi_scale_deformable_attn_softmax
 from muspace_amd.ops.scatter_div import multi_scale_deformable_attn_scatter_div
+from muspace_amd.runtime.native import load_native_module
 from oracle import msda_torch
 
 pytestmark = [
@@ -64,15 +65,16 @@ def _compare(actual, expected):
 F32, F16, BF16 = torch.float32, torch.float16, torch.bfloat16
 CASES = [
     # (levels, queries, points, heads, channels, batch, value, geometry): what is kept in LDS
-    (((30, 40), (15, 20), (8, 10), (4, 5)), 4100, 8, 8, 32, 1, F32, F32),  # the last three levels
+    (((30, 40), (15, 20), (8, 10), (4, 5)), 5921, 8, 8, 32, 1, F32, F32),  # the last three levels
     (((12, 16), (6, 8), (3, 4), (2, 2)), 8200, 4, 8, 32, 1, F32, F32),     # every level
     (((90, 100), (70, 80)), 8201, 8, 8, 32, 1, F32, F32),                  # none
     (((4, 5), (8, 10), (60, 70)), 5500, 8, 8, 32, 1, F32, F32),            # none: fine level last
     (((60, 70), (30, 35), (1, 1), (1, 2)), 6600, 5, 8, 32, 1, F32, F32),   # 20 samples
     (((60, 70), (30, 35), (15, 18)), 15000, 3, 8, 32, 1, F32, F32),        # 9 samples: ragged stages
-    (((60, 70), (30, 35)), 33000, 2, 8, 32, 1, F32, F32),                  # 4 samples
-    (((40, 50), (20, 25), (10, 13), (5, 7)), 4100, 8, 8, 32, 1, BF16, F32),
-    (((40, 50), (20, 25), (10, 13), (5, 7)), 4133, 8, 8, 32, 1, F16, F16),
+    (((60, 70), (30, 35)), 32768, 2, 8, 32, 1, F32, F32),                  # 4 samples, whole rounds
+    (((60, 70), (30, 35)), 33000, 2, 8, 32, 1, F16, F32),                  # 4 samples
+    (((40, 50), (20, 25), (10, 13), (5, 7)), 7650, 8, 8, 32, 1, BF16, F32),
+    (((40, 50), (20, 25), (10, 13), (5, 7)), 7999, 8, 8, 32, 1, F16, F16),
     (((60, 70), (30, 35), (15, 18)), 7500, 4, 8, 32, 3, F16, F32),         # 12 samples
     (((60, 70), (30, 35), (15, 18)), 15000, 3, 8, 32, 1, BF16, BF16),      # 9 samples, 16-bit pairs
     (((40, 50), (20, 25), (10, 13), (5, 7)), 8300, 8, 4, 64, 1, F32, F32),
@@ -90,6 +92,8 @@ def test_matches_the_row_kernel_and_the_oracle(case):
     value, shapes, starts, loc, logits = _inputs(5, levels, queries, points, heads, channels,
                                                  batch, vdt, gdt)
     attn = _weights(logits, gdt)
+    lib = load_native_module()
+    assert lib.forward_takes_slab(value, loc) and not lib.forward_takes_slab(value, loc[:, :PIECE])
     out = multi_scale_deformable_attn(value, shapes, starts, loc, attn)
     _compare(out, _by_rows(value, shapes, starts, loc, attn))
     pick = torch.arange(0, queries, queries // 40)
@@ -104,8 +108,9 @@ def test_matches_the_row_kernel_and_the_oracle(case):
 @pytest.mark.parametrize("vdt", [F32, F16])
 def test_bad_levels_contribute_nothing(vdt):
     """A level past the value and one that overlaps another, among the LDS levels."""
-    value, shapes, starts, loc, logits = _inputs(6, ((30, 40), (15, 20), (8, 10), (4, 5)), 4100, 8,
+    value, shapes, starts, loc, logits = _inputs(6, ((30, 40), (15, 20), (8, 10), (4, 5)), 7900, 8,
                                                  vdt=vdt)
+    assert load_native_module().forward_takes_slab(value, loc)
     starts = starts.clone()
     starts[2] = 1200  # inside level 1
     starts[3] = value.shape[1] - 3
@@ -115,12 +120,16 @@ def test_bad_levels_contribute_nothing(vdt):
 
 
 @pytest.mark.parametrize("vdt", [F32, BF16])
-@pytest.mark.parametrize("lens", [(4300, 4300, 4100), (4300, 0, 17)])
-def test_camera_average(vdt, lens):
-    """Cameras of unequal length (one empty) into BEV slots, an index out of range."""
-    cams, nq = len(lens), 6000
-    value, shapes, starts, loc, logits = _inputs(7, ((30, 40), (15, 20), (8, 10), (4, 5)), 4300, 8,
-                                                 batch=cams, vdt=vdt)
+@pytest.mark.parametrize("lens", [(7900, 7900, 7600), (7900, 0, 17)])
+@pytest.mark.parametrize("levels", [((30, 40), (15, 20), (8, 10), (4, 5)), ((30, 40),)],
+                         ids=["four", "one"])
+def test_camera_average(vdt, lens, levels):
+    """Cameras of unequal length (one empty) into BEV slots, an index out of range.
+    With one level cameras keep the row kernel."""
+    cams, nq = len(lens), 9000
+    value, shapes, starts, loc, logits = _inputs(7, levels, 7900, 8, batch=cams, vdt=vdt)
+    assert (load_native_module().forward_takes_slab(value[:1], loc[:1, : max(lens)], cams)
+            == (len(levels) > 1))
     attn = _weights(logits, F32)
     g = torch.Generator().manual_seed(8)
     indexes = [torch.randperm(nq, generator=g)[:n].to(DEV) for n in lens]
@@ -170,9 +179,9 @@ def test_records_past_the_memory_side_cache():
     """A batch whose binned records pass 256 MB (their stores then go through the L2)
     gives what its entries give one by one. Outputs and location and weight
     gradients are each one unit's or sample's own sum. A value gradient sums, in
-    another order, up to some 350 products (23000 queries x 4 samples x 4 corners over
-    1050 cells) whose magnitudes add up to about 9: 350 * 2^-24 * 9 = 1.9e-4 at worst."""
-    levels, queries, points, batch = ((60, 70), (30, 35)), 23000, 4, 12
+    another order, up to some 350 products (20200 queries x 4 samples x 4 corners over
+    952 cells) whose magnitudes add up to about 9: 350 * 2^-24 * 9 = 1.9e-4 at worst."""
+    levels, queries, points, batch = ((56, 68), (28, 34)), 20200, 4, 13
     value, shapes, starts, loc, logits = _inputs(11, levels, queries, points, batch=batch)
     assert batch * queries * 8 * len(levels) * points * 16 > 256 << 20
     attn = _weights(logits, F32)
