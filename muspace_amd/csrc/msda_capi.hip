@@ -162,17 +162,19 @@ Launch plan_rows(const msda::Shape &s, int kq, int max_ns, bool forward) {
   const int64_t per_block = msda::kBlock / msda::kWave;
   // units per lane group: 8 (the next unit's geometry loads overlap the
   // gathers, and a block's prologue is shared by more units), fewer where 8
-  // would leave the 256 CUs short of two blocks each. Measured at 8 and as
+  // would leave the 256 CUs far short of two blocks each. Measured at 8 and as
   // chosen: 1000 queries x 8 heads x 16 samples fp32 (63 -> 500 blocks) 15.1 ->
   // 7.5 us, 300 queries fp16 14.3 -> 5.4 us, the fused binning forward at 2 x
   // 900 queries 31.2 -> 17.5 us (its bin_count 14.1 -> 9.1 us). Where 8 fills
   // the chip already, fewer is slower: 2 x 22223 queries 196 us at 8, 210 at 4,
-  // 252 at 2.
+  // 252 at 2; and from 400 blocks on half as many units a group make a second,
+  // nearly empty round: 436 blocks 175 us, 871 blocks 185 (six cameras of 3481
+  // bf16 rows); 428 blocks 113 us, 856 blocks 119.
   L.plan.iters = 8;
   do {
     const int64_t waves = (wave_iters + L.plan.iters - 1) / L.plan.iters;
     L.blocks = static_cast<int>((waves + per_block - 1) / per_block);
-    if (L.blocks >= 512 || L.plan.iters == 1) break;
+    if (L.blocks >= 400 || L.plan.iters == 1) break;
     L.plan.iters /= 2;
   } while (true);
   return L;

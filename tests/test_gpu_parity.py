@@ -427,6 +427,20 @@ def test_value_past_2gib_takes_the_wide_paths(native_lib, path):
         _assert_close(ga[sl], o_ga, 1e-4, f"grad_attention_weights[{b}]")
 
 
+@pytest.mark.parametrize("queries", [1597, 1600, 3184, 3200, 6383, 6400])
+def test_row_kernel_units_per_group(native_lib, queries):
+    """Around 400 blocks at two, four and eight units per lane group: a unit's sums do
+    not depend on the grouping, so parts of 97 queries (one unit a group) give the
+    same bits."""
+    t, _ = small_case(29, 1, queries, 8, 32, ((9, 13), (5, 4)), 8)
+    whole = run_forward(native_lib, t, torch.float32, torch.float32)
+    for q in range(0, queries, 97):
+        part = dict(t, sampling_locations=t["sampling_locations"][:, q:q + 97],
+                    attention_weights=t["attention_weights"][:, q:q + 97])
+        out = run_forward(native_lib, part, torch.float32, torch.float32)
+        assert torch.equal(whole[:, q:q + 97], out)
+
+
 @pytest.mark.parametrize("path", ["one_call", "fused"])
 @pytest.mark.parametrize("levels", [((200, 200), (100, 95)), ((200, 200), (100, 100)),
                                     ((206, 206), (103, 100)), ((215, 215), (107, 100))])
