@@ -241,6 +241,7 @@ struct SlabLaunch {
   bool wide = false;    // several samples per geometry load
   bool coarse = false;  // a level in LDS, if the levels are a pyramid
   bool ragged = false;  // the row kernel's steps are less than 9/10 full
+  double score = 0.0;   // how full the slab kernel runs against the row kernel
   msda::SlabPlan plan{};
 };
 
@@ -334,12 +335,12 @@ SlabLaunch plan_slab(const msda::Shape &s, int64_t slabs, int queries, size_t el
   const int places = (L.plan.chunk_q + round - 1) / round * round;
   const double queries_full = static_cast<double>(L.plan.chunk_q) / places;
   const double samples_full = static_cast<double>(s.lp) / ((s.lp + ns - 1) / ns * ns);
-  const double score = queries_full * queries_full * samples_full / rows_full;
+  L.score = queries_full * queries_full * samples_full / rows_full;
   if (cameras && elem == 2) {
-    L.ok = score >= 0.5 && L.coarse;
+    L.ok = L.score >= 0.5 && L.coarse;
     return L;
   }
-  L.ok = score >= (elem == 2 ? 0.74 : 0.5) &&
+  L.ok = L.score >= (elem == 2 ? 0.74 : 0.5) &&
          (chunks == per_slab || lines <= (elem == 2 ? 2000000 : 4200000) ||
           (chunks % per_slab == 0 && lines <= 4200000)) &&
          (!cameras || L.coarse || L.ragged);
@@ -1046,7 +1047,9 @@ bool fwd_bin_fuses(const msda::Shape &s, int value_dtype, const TileWorkspace &w
 // binning kernels' scatter pays more for: 159 us).
 //
 // The slab forward has to win by more than the scatter costs: with a level in LDS,
-// or against ragged steps of the row kernel in float32 (586 drawn shapes: 67 below
+// or against ragged steps of the row kernel in float32, and nearly full rounds in
+// either width (8162 queries of 6 heads, 25 samples fp32: 142 us with the records
+// stored by the row kernel, 153 apart at a score of 0.58; 586 drawn shapes: 67 below
 // 0.98 where only plan_slab decides, down to 0.88; with this rule 5 of 375, the lowest
 // 0.96, geometric mean 1.09). One level: float32 from 80 chunks of 1200 samples on
 // (27 drawn shapes 1.00 to 1.16; BEVFormer's 200 x 200, 2 x 40000 queries, 298 -> 291
@@ -1059,7 +1062,7 @@ bool bins_apart(const msda::Shape &s, size_t elem) {
   if (L.narrow) {
     return elem == 4 && slab_chunks(L, s.queries) >= 80 && L.plan.chunk_q * s.lp >= 1200;
   }
-  return L.coarse || (elem == 4 && L.ragged);
+  return L.score >= 0.74 && (L.coarse || (elem == 4 && L.ragged));
 }
 
 // The forward with the backward's binning fused in (msda_forward_bin.hpp):
