@@ -203,11 +203,11 @@ MUSPACE_API int ms_deform_attn_forward_slab(int value_dtype, int64_t num_cams, i
 
 /* 1 if the forward kernel of ms_deform_attn_forward_bin, given 16-byte-aligned
  * tensors and a 256-byte-aligned workspace of
- * ms_deform_attn_backward_workspace_size bytes, can store the backward's
- * records for these dims (large shapes take the other form all the same, where
- * it is faster); 0 if the call runs ms_deform_attn_forward and the binning
- * kernels (or the shape takes the atomic backward). Results are the same
- * either way. No reference counterpart. */
+ * ms_deform_attn_backward_workspace_size bytes, stores the backward's records
+ * for these dims; 0 if the call runs the binning kernels and
+ * ms_deform_attn_forward, because that is faster or the only form (or the shape
+ * takes the atomic backward). Results are the same either way. No reference
+ * counterpart. */
 MUSPACE_API int ms_deform_attn_forward_bin_fused(int value_dtype, int64_t batch,
                                                  int64_t spatial_size, int64_t num_heads,
                                                  int64_t channels, int64_t num_levels,
@@ -351,9 +351,10 @@ MUSPACE_API int ms_deform_attn_forward_softmax_bin(
     size_t workspace_bytes, void *stream);
 
 /* 1 if ms_deform_attn_forward_softmax_bin (aligned tensors, a workspace as
- * above) can fuse the probabilities and the record stores into the forward
- * kernel for these dims (large shapes take the other form where it is faster);
- * 0 if it makes the two calls. No reference counterpart. */
+ * above, geometry of the value's type) fuses the probabilities and the record
+ * stores into the forward kernel for these dims; 0 if it makes the two calls.
+ * With a 16-bit value and float32 geometry it fuses them where
+ * ms_deform_attn_forward_bin_fused is 1 as well. No reference counterpart. */
 MUSPACE_API int ms_deform_attn_forward_softmax_bin_fused(int value_dtype, int64_t batch,
                                                          int64_t spatial_size,
                                                          int64_t num_heads, int64_t channels,

@@ -1568,7 +1568,8 @@ int ms_deform_attn_forward_bin_fused(int value_dtype, int64_t batch, int64_t spa
   TileWorkspace w;
   int units = 0, slots = 0;
   return needs_data(s) && s.lp > 0 && plan_tile_workspace(s, value_dtype, w) &&
-                 fwd_bin_fuses(s, value_dtype, w, units, slots)
+                 fwd_bin_fuses(s, value_dtype, w, units, slots) &&
+                 !bins_apart(s, value_dtype == MUSPACE_DTYPE_F32 ? 4 : 2)
              ? 1
              : 0;
 }
@@ -1914,8 +1915,10 @@ int ms_deform_attn_forward_softmax_bin_fused(int value_dtype, int64_t batch,
   ok();
   TileWorkspace w;
   int units = 0, slots = 0;
+  // with 16-bit geometry the probabilities stay in the forward kernel
   return needs_data(s) && s.lp > 0 && plan_tile_workspace(s, value_dtype, w) &&
-                 fwd_bin_fuses(s, value_dtype, w, units, slots, true)
+                 fwd_bin_fuses(s, value_dtype, w, units, slots, true) &&
+                 !(value_dtype == MUSPACE_DTYPE_F32 && bins_apart(s, 4))
              ? 1
              : 0;
 }

@@ -531,10 +531,9 @@ class NativeLibrary:
             points))
 
     def forward_bin_fuses(self, value, sampling_locations) -> bool:
-        """Whether the forward kernel of :meth:`ms_deform_attn_forward_bin` can
-        store the backward's records for these shapes (it does where that is
-        the faster form; else the call runs the plain forward and the binning
-        kernels; same results)."""
+        """Whether the forward kernel of :meth:`ms_deform_attn_forward_bin`
+        stores the backward's records for these shapes (else the call runs the
+        binning kernels and the plain forward; same results)."""
         batch, spatial, heads, channels = value.shape
         _, queries, _, levels, points, _ = sampling_locations.shape
         return bool(self._raw["ms_deform_attn_forward_bin_fused"](
@@ -542,10 +541,12 @@ class NativeLibrary:
 
     def forward_softmax_bin_fuses(self, value, sampling_locations) -> bool:
         """Whether the softmax-fused forward kernel of
-        :meth:`ms_deform_attn_forward_softmax_bin` can write the probabilities
-        and store the backward's records for these shapes (it does where that
-        is the faster form; else the call runs a forward and the softmax
-        binning; same results)."""
+        :meth:`ms_deform_attn_forward_softmax_bin` writes the probabilities and
+        stores the backward's records for these shapes and types (else the call
+        runs a forward and the softmax binning; same results)."""
+        if sampling_locations.dtype != value.dtype and not self.forward_bin_fuses(
+                value, sampling_locations):
+            return False
         batch, spatial, heads, channels = value.shape
         _, queries, _, levels, points, _ = sampling_locations.shape
         return bool(self._raw["ms_deform_attn_forward_softmax_bin_fused"](

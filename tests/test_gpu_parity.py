@@ -544,8 +544,45 @@ def test_full_config_parity(native_lib, name, value_dtype, geometry_dtype):
     _check_full_config(native_lib, name, value_dtype, geometry_dtype, fused=False)
 
 
-# The fused forward + binning at full size, at every config the bench times
-# through it: float32 (c1, c2, c3) and both 16-bit value types (c4).
+# Large shapes whose forward kernel stores the records: float32 without a level in
+# LDS, one float32 level of few chunks, and 16-bit shapes without a level in LDS.
+LARGE_STORED = [
+    (torch.float32, 2, 20000, ((90, 100), (70, 80)), 8),
+    (torch.float32, 5, 16000, ((100, 100),), 4),
+    (torch.bfloat16, 2, 20000, ((90, 100), (70, 80)), 5),
+    (torch.float16, 2, 40000, ((100, 100),), 4),
+]
+
+
+@pytest.mark.parametrize("value_dtype,batch,queries,levels,points", LARGE_STORED, ids=[
+    f"{str(c[0])[6:]}-b{c[1]}-q{c[2]}-{len(c[3])}x{c[4]}" for c in LARGE_STORED])
+def test_records_stored_by_the_forward_at_large_shapes(native_lib, value_dtype, batch, queries,
+                                                       levels, points):
+    """Against the binning kernels' records (a backward of its own) and, on a subset
+    of the queries, the oracle. Location and weight gradients are each one sample's
+    own sums; a value gradient sums the same products in another order."""
+    t, grad = small_case(37, batch, queries, 8, 32, levels, points)
+    assert native_lib.forward_bin_fuses(t["value"].to(value_dtype), t["sampling_locations"])
+    out, gv, gl, ga = run_fused(native_lib, t, grad, value_dtype, torch.float32)
+    b_gv, b_gl, b_ga = run_backward(native_lib, t, grad, value_dtype, torch.float32)
+    ftol, btol = TOL[value_dtype]
+    for got, ref, what in ((gv, b_gv, "grad_value"), (gl, b_gl, "grad_sampling_locations"),
+                           (ga, b_ga, "grad_attention_weights")):
+        _assert_close(got, ref, btol, what)
+    idx = torch.arange(0, queries, queries // SUBSET)
+    value, shapes, loc, attn = oracle_inputs(t, value_dtype, torch.float32)
+    gq = grad.to(value_dtype).float()
+    o_out, _, o_gl, o_ga = msda_torch.msda_forward_backward(value, shapes, loc[:, idx],
+                                                            attn[:, idx], gq[:, idx])
+    _assert_close(out.cpu()[:, idx], o_out, ftol, "output (query subset)")
+    _assert_close(gl.cpu()[:, idx], o_gl, btol, "grad_sampling_locations (query subset)")
+    _assert_close(ga.cpu()[:, idx], o_ga, btol, "grad_attention_weights (query subset)")
+
+
+# The forward + binning call at full size, at every config the bench times through
+# it: float32 (c1, c2, c3) and both 16-bit value types (c4). At c2 the forward
+# kernel stores the records, at the others the binning kernels run before the
+# forward that keeps a slab's coarse levels in LDS.
 FULL_FUSED = [
     ("c1", torch.float32, torch.float32),
     ("c2", torch.float32, torch.float32),
@@ -553,6 +590,7 @@ FULL_FUSED = [
     ("c4", torch.bfloat16, torch.float32),
     ("c4", torch.float16, torch.float32),
 ]
+STORES_RECORDS = {"c2"}
 
 
 @pytest.mark.parametrize("name,value_dtype,geometry_dtype", FULL_FUSED,
@@ -568,9 +606,8 @@ def _check_full_config(native_lib, name, value_dtype, geometry_dtype, fused):
     t = make_inputs(cfg, value_dtype=torch.float32)
     grad = t.pop("grad_output")
     if fused:
-        # the forward kernel itself stores the records here (no fallback to
-        # the binning kernels)
-        assert native_lib.forward_bin_fuses(t["value"].to(value_dtype), t["sampling_locations"])
+        stores = native_lib.forward_bin_fuses(t["value"].to(value_dtype), t["sampling_locations"])
+        assert stores == (name in STORES_RECORDS)
         out, gv, gl, ga = run_fused(native_lib, t, grad, value_dtype, geometry_dtype)
         plain = run_forward(native_lib, t, value_dtype, geometry_dtype)
         torch.cuda.synchronize()
