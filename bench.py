@@ -501,8 +501,9 @@ def time_dfa(lib, steps: int = 50, warmup: int = 10) -> dict:
     scope as the reference's benchmark
     (/root/reference/benchmarks/deformable_aggregation/README.md:31-40): output
     and gradients allocated once before the timed region, one entry-point call
-    per launch (the kernels add into those buffers, which changes the values,
-    not the work)."""
+    each, the ones that the operator makes (the forward adds into its buffer,
+    which changes the values, not the work; the backward overwrites the
+    gradients, its scratch from torch's caching allocator)."""
     t = make_dfa_inputs(device="cuda")
     mc, spatial, start = t["mc_ms_feat"], t["spatial_shape"], t["scale_start_index"]
     loc, weights, grad = t["sampling_location"], t["weights"], t["grad_output"]
@@ -510,7 +511,7 @@ def time_dfa(lib, steps: int = 50, warmup: int = 10) -> dict:
     gf, gl, gw = torch.zeros_like(mc), torch.zeros_like(loc), torch.zeros_like(weights)
     fwd_ms = _event_ms(lambda: lib.deformable_aggregation_forward_opt(
         mc, spatial, start, loc, weights, out), steps, warmup)
-    bwd_ms = _event_ms(lambda: lib.deformable_aggregation_backward_opt(
+    bwd_ms = _event_ms(lambda: lib.deformable_aggregation_backward(
         mc, spatial, start, loc, weights, grad, gf, gl, gw), steps, warmup)
     fwd_b, bwd_b = dfa_algorithmic_bytes()
     active = float(((loc > 0) & (loc < 1)).all(-1).float().mean())
