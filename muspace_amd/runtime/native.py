@@ -264,6 +264,7 @@ class NativeLibrary:
             )
         # scratch sizes by device and dims (a plan each, asked for several times a step)
         self._size = lru_cache(maxsize=1024)(self._workspace_size)
+        self._dfa_scratch = lru_cache(maxsize=1024)(self._dfa_scratch_bytes)
         self._bound: dict[str, Callable[..., Any]] = {
             "check_forward": self.check_forward,
             "check_backward": self.check_backward,
@@ -893,6 +894,13 @@ class NativeLibrary:
             sampling_location.data_ptr(), weights.data_ptr(), output.data_ptr(), *dims,
         )
 
+    def _dfa_scratch_bytes(self, *dims) -> int:
+        """Scratch of the aggregation's backward for these dims, 0 where the
+        kernels without are the faster ones."""
+        if not self._raw["deformable_aggregation_backward_prefers_workspace"](*dims):
+            return 0
+        return int(self._raw["deformable_aggregation_backward_workspace_size"](*dims))
+
     def _dfa_backward(self, name, mc_ms_feat, spatial_shape, scale_start_index,
                       sampling_location, weights, grad_output, grad_mc_ms_feat,
                       grad_sampling_location, grad_weights, with_workspace=False) -> None:
@@ -907,8 +915,8 @@ class NativeLibrary:
             _check(tensor, label, (torch.float32,))
             _check_shape(tensor, label, like)
         scratch = (None, 0) if with_workspace else ()
-        if with_workspace and self._raw["deformable_aggregation_backward_prefers_workspace"](*dims):
-            nbytes = self._raw["deformable_aggregation_backward_workspace_size"](*dims)
+        nbytes = self._dfa_scratch(*dims) if with_workspace else 0
+        if nbytes:
             try:
                 workspace = torch.empty(nbytes, dtype=torch.uint8, device=mc_ms_feat.device)
                 scratch = (workspace.data_ptr(), nbytes)
