@@ -273,10 +273,10 @@ double row_fill(const msda::Shape &s, size_t elem) {
 // Workgroups of eight wavefronts, one a CU, in whole rounds over the 256 CUs. An
 // XCD's 32 CUs work on neighbouring chunks, so 32 chunks a slab keep it on one
 // slab, whose lines its L2 holds; where two heads share a 128-byte line (rows of
-// 64 bytes), 16 keep it on two heads' slabs. At the SCA shape fp32 took 579, 412,
-// 325 and 385 us at 8, 16, 32 and 48 chunks, bf16 227, 275 and 309 at 16, 32 and
-// 48; 3 x 8 slabs of 10007 fp16 queries 60 us at 16 (a round and a half), 54 at
-// 20. A workgroup copies the coarse levels (up to 119 KB) first, which takes 4096
+// 64 bytes), 16 keep it on two heads' slabs. The kernel alone with warm values, at
+// the SCA shape: fp32 579, 412, 325 and 385 us at 8, 16, 32 and 48 chunks, bf16 227,
+// 275 and 309 at 16, 32 and 48; 3 x 8 slabs of 10007 fp16 queries 60 us at 16 (a
+// round and a half), 54 at 20. A workgroup copies the coarse levels (up to 119 KB) first, which takes 4096
 // samples to pay for. With one level there is nothing to copy, and workgroups of
 // four wavefronts and about 2048 of them are best (200 x 200 cells, 2 x 40000
 // queries, fp32: 83 us; eight wavefronts: 112, 94 and 88 us at 32, 48 and 64

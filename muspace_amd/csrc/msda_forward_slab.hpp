@@ -15,13 +15,16 @@
 // queries, a pass computes the taps of NS samples of each, one per lane, and a
 // stage gathers and sums NH of them. No sums over lane groups are left.
 //
-// Measured against the row kernel, value warm (8 heads x 32 channels; the LDS
-// levels' share of the samples in brackets): the SCA shape (6 x 10000 queries, 4
+// Measured against the row kernel, the kernel alone over and over with its value
+// warm in the caches (8 heads x 32 channels; the LDS levels' share of the samples in
+// brackets): the SCA shape (6 x 10000 queries, 4
 // levels x 8 points) fp32 [1/4] 365 -> 325 us, bf16 [1/2] 313 -> 227 us; twice
 // the batch, 15000 queries, bf16 860 -> 697 us; the encoder shape (2 x 22223, 4
 // levels x 4 points) fp32 [1/4] 145 -> 99 us, fp16 [1/2] 105 -> 78 us; 3 x 10007
 // queries on three levels, fp16 [2/3] 73 -> 52 us; one 200 x 200 level (no LDS
-// level; 4 wavefronts a workgroup) fp32 106 -> 83 us, bf16 93 -> 72 us. What is
+// level; 4 wavefronts a workgroup) fp32 106 -> 83 us, bf16 93 -> 72 us. In a program's
+// calls, with other inputs and other kernels between, it takes 246 us at the bf16 SCA
+// shape, 746 at twice the batch, 117 at the encoder and 105 on the one level. What is
 // left is the fine levels' gathers from L2 (46 M lines in 325 us at the SCA
 // shape in fp32), and in bf16 the decode and multiply-adds (about 137 us of VALU
 // there). On the way: geometry loads marked non-temporal cost 4-30% (a pass
@@ -262,7 +265,9 @@ __global__ void __launch_bounds__(W * kWave, kRowWavesPerSimd)
   // float32 sums a unit in four chains (by pass parity and stage), as long as
   // those of the row kernel's lane groups; one chain of a unit's 32 samples
   // raised the error against 64 bits from 8.4e-8 to 1.2e-7. In 16 bits the
-  // result's own rounding is 2e-4 and more.
+  // result's own rounding is 2e-4 and more: with two chains the error against 64
+  // bits agrees in five digits at 256 samples a unit (fp16 2.0795e-4, bf16
+  // 1.6583e-3).
   constexpr int kChains = std::is_same<VT, float>::value ? 2 * TS : 1;
   float acc[kChains][CPL];
 #pragma unroll
